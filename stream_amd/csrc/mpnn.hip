@@ -374,14 +374,45 @@ __global__ __launch_bounds__(256) void gemm_dw_kernel(uint32_t n, uint32_t rows_
     }
 }
 
-__global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ partial, uint32_t nblk,
-                                                              uint32_t stride, uint32_t width,
-                                                              float* __restrict__ dst) {
-    const uint32_t o = blockIdx.x * 256 + threadIdx.x;
-    if (o >= width) return;
+// dst[o] = the FP64 sum over the nblk block partials of column o, 16 columns
+// per block of 1024 threads.  Bound: the latency of the row loads (the
+// partials are a few MB in the caches), so 64 rows of a column are summed
+// side by side (a 64-byte run of a row per 16 lanes) with 4 rows per thread in
+// flight; one thread per column walking all rows in turn took 250 us per
+// launch for 65k nodes, two thirds of the gradient.  Fixed order: rows r,
+// r + 64, ... per lane, then the wave's 4 lanes, then the waves.
+constexpr uint32_t kRedCols = 16, kRedLanes = 64;
+__global__ __launch_bounds__(1024) void reduce_partials_kernel(const float* __restrict__ partial, uint32_t nblk,
+                                                               uint32_t width, float* __restrict__ dst) {
+    __shared__ double sw[16][kRedCols];
+    const uint32_t c = threadIdx.x % kRedCols, rl = threadIdx.x / kRedCols;
+    const uint32_t o = blockIdx.x * kRedCols + c;
     double s = 0.0;
-    for (uint32_t b = 0; b < nblk; ++b) s += partial[(size_t)b * stride + o];
-    dst[o] = (float)s;
+    if (o < width) {
+        uint32_t b = rl;
+        for (; b + 3 * kRedLanes < nblk; b += 4 * kRedLanes) {
+            float v[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) v[u] = partial[(size_t)(b + u * kRedLanes) * width + o];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) s += v[u];
+        }
+        for (; b < nblk; b += kRedLanes) s += partial[(size_t)b * width + o];
+    }
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if ((threadIdx.x & 63u) < kRedCols) sw[threadIdx.x >> 6][c] = s;
+    __syncthreads();
+    if (threadIdx.x < kRedCols && o < width) {
+        double t = 0.0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) t += sw[w][c];
+        dst[o] = (float)t;
+    }
+}
+void reduce_partials(const float* partial, uint32_t nblk, uint32_t width, float* dst, hipStream_t s) {
+    hipLaunchKernelGGL(reduce_partials_kernel, dim3((width + kRedCols - 1) / kRedCols), dim3(1024), 0, s, partial, nblk,
+                       width, dst);
 }
 
 // ---------------------------------------------------------------------------
@@ -879,8 +910,7 @@ void run_dw(uint32_t n, const float* x0, uint32_t ld0, const float* x1, uint32_t
     const uint32_t width = K * N + (BIAS ? N : 0);
     hipLaunchKernelGGL((gemm_dw_kernel<K, K0, N, BIAS>), dim3(nb), dim3(256), 0, s, n, rpb, x0, ld0, x1, ld1, dy,
                        lddy, partial);
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((width + 255) / 256), dim3(256), 0, s, partial, nb, width,
-                       width, dst);
+    reduce_partials(partial, nb, width, dst, s);
 }
 
 }  // namespace
@@ -1007,8 +1037,7 @@ void MpnnNet::backward(const MpnnGraph& g, hipStream_t s) {
     float* G = grad.p;
     hipLaunchKernelGGL(head_bwd_kernel, dim3(eg), dim3(256), 0, s, n, g.row, g.col, g.val, g.dpos.p, g.tr.p, g.bnd,
                        g.efeat.p, RSD.p, wb.p, w.p, gval.p, od.p, y.p, lsc.p, dRSD.p, partials.p);
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((kHeadPart + 255) / 256), dim3(256), 0, s, partials.p, eg,
-                       kHeadPart, kHeadPart, G + kParams.de_w);
+    reduce_partials(partials.p, eg, kHeadPart, G + kParams.de_w, s);
     run_dw<64, 64, 192, false>(n, H[kLayers].p, kHid, nullptr, 0, dRSD.p, kRsd, partials.p, G + kParams.dec_w, s);
     // dH3 = dRSD W_dec^T
     run_gemm<192, 192, 64, kEpiAdd>(gargs(n, dRSD.p, kRsd, wb.p + kParams.dec_w, dHa.p, kHid), s);
@@ -1023,8 +1052,7 @@ void MpnnNet::backward(const MpnnGraph& g, hipStream_t s) {
         run_gemm<64, 64, 128, kEpiStore>(gargs(n, dU.p, kHid, wb.p + kParams.u_w[l], dX.p, kPq), s);
         hipLaunchKernelGGL(msg_bwd_kernel, dim3(eg), dim3(256), 0, s, n, g.row, g.col, g.efeat.p, g.deg.p,
                            PQ[l].p, dX.p, wb.p, w.p, (uint32_t)l, dPQ.p, partials.p);
-        hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, s, partials.p, eg, kMsgPart, kMsgPart,
-                           G + kParams.e_w[l]);
+        reduce_partials(partials.p, eg, kMsgPart, G + kParams.e_w[l], s);
         run_dw<64, 64, 128, false>(n, H[l].p, kHid, nullptr, 0, dPQ.p, kPq, partials.p, G + kParams.pq_w[l], s);
         // dH_l = dH_{l+1} + dX[:, :64] + dPQ W_pq^T
         GemmArgs a = gargs(n, dPQ.p, kPq, wb.p + kParams.pq_w[l], dh_next, kHid);
@@ -1039,8 +1067,7 @@ void MpnnNet::backward(const MpnnGraph& g, hipStream_t s) {
     }
     const unsigned encg = blocks_for(n, 4, kEdgeGrid);
     hipLaunchKernelGGL(enc_bwd_kernel, dim3(encg), dim3(256), 0, s, n, g.nfeat.p, H[0].p, dh, partials.p);
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((kEncPart + 255) / 256), dim3(256), 0, s, partials.p, encg,
-                       kEncPart, kEncPart, G + kParams.enc_w);
+    reduce_partials(partials.p, encg, kEncPart, G + kParams.enc_w, s);
 }
 
 void MpnnNet::adam(float lr, float b1, float b2, float eps, hipStream_t s) {
