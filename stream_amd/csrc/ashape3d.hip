@@ -158,31 +158,135 @@ template <class S> __device__ __forceinline__ void load3(const Sph4<S>* P, uint3
     p[2] = s.c[2];
 }
 
-// Local Delaunay of node tid's star + alpha filter (cpp:380-682).
-// EXACT = false returns false at the first insphere whose filter cannot
-// certify the sign; the node is then redone by the exact kernel.
-template <class S, bool EXACT>
-__device__ bool local_delaunay3(const Ash3Args<S>& a, uint32_t tid, uint8_t* cyc, double* ws) {
+// Boundary of the R removed tetrahedra at positions Tlast .. Tlast + R - 1 of
+// T (cpp:497-580): Ray et al.'s cycle walk, C(v) = next vertex of v on the
+// cycle (kEmpty off it).  C must be kEmpty for every vertex of the star.
+// Returns true when the 100-step cap stopped the walk (an open star);
+// *first_out is the vertex that the re-triangulation starts from.
+template <class TF, class CF>
+__device__ __forceinline__ bool cavity_walk(TF&& T, CF&& C, uint32_t Tlast, uint32_t Rsize, uint32_t* first_out) {
+    --Rsize;
+    const uint32_t tlst = T(Tlast + Rsize);
+    const uint32_t ta = tlst & 255u, tb = (tlst >> 8) & 255u, tc3 = (tlst >> 16) & 255u;
+    C(ta) = tb;
+    C(tb) = tc3;
+    C(tc3) = ta;
+    uint32_t cur = Tlast;
+    uint32_t first = ta;
+    int swap_with = (int)(Tlast + Rsize) - 1;
+    uint32_t failed = 0;
+    int niter = 0;
+    while (Rsize && niter++ < 100) {
+        const uint32_t tw = T(cur);
+        const uint32_t tcv[3] = {tw & 255u, (tw >> 8) & 255u, (tw >> 16) & 255u};
+        const uint32_t ty[3] = {C(tcv[0]), C(tcv[1]), C(tcv[2])};
+        bool inb[3], opp[3];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            inb[e] = ty[e] != kEmpty;
+            opp[e] = ty[(e + 1) % 3] == tcv[e];
+        }
+        bool simple = opp[0] || opp[1] || opp[2];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) simple &= (opp[e] || opp[(e + 1) % 3] || !inb[(e + 1) % 3]);
+        if (!simple) {
+            // a pass in which all fail leaves the rest of the steps to fail too
+            if (++failed == Rsize) break;
+            ++cur;
+            continue;
+        }
+        failed = 0;
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            if (!opp[e]) C(tcv[e]) = tcv[(e + 1) % 3];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            if (opp[e] && opp[(e + 1) % 3]) {
+                if (first == tcv[(e + 1) % 3]) first = ty[(e + 1) % 3];
+                C(tcv[(e + 1) % 3]) = kEmpty;
+            }
+        }
+        T(cur) = T((uint32_t)swap_with);
+        T((uint32_t)swap_with) = tw;
+        --swap_with;
+        --Rsize;
+        cur = Tlast;
+    }
+    *first_out = first;
+    return Rsize != 0;
+}
+
+// The alpha filter of the tetrahedron (tid, i2, i3, i4) (cpp:590-682): kept
+// when its squared circumradius is at most every corner's alpha^2; *own when
+// tid is its lowest id.
+template <class S>
+__device__ __forceinline__ bool alpha_keep(const Sph4<S>* P, uint32_t tid, uint32_t i2, uint32_t i3, uint32_t i4,
+                                           bool* own) {
+    uint32_t i1 = tid, t;
+    if (i1 > i3) { t = i3; i3 = i1; i1 = t; }
+    if (i2 > i4) { t = i4; i4 = i2; i2 = t; }
+    if (i1 > i2) { t = i2; i2 = i1; i1 = t; }
+    if (i3 > i4) { t = i4; i4 = i3; i3 = t; }
+    if (i2 > i3) { t = i3; i3 = i2; i2 = t; }
+    const Sph4<S> qa = P[i1], qb = P[i2], qc = P[i3], qd = P[i4];
+    const S tv[3] = {qa.c[0] - qd.c[0], qa.c[1] - qd.c[1], qa.c[2] - qd.c[2]};
+    const S uv[3] = {qb.c[0] - qd.c[0], qb.c[1] - qd.c[1], qb.c[2] - qd.c[2]};
+    const S vv[3] = {qc.c[0] - qd.c[0], qc.c[1] - qd.c[1], qc.c[2] - qd.c[2]};
+    const S d2t = tv[0] * tv[0] + tv[1] * tv[1] + tv[2] * tv[2];
+    const S d2u = uv[0] * uv[0] + uv[1] * uv[1] + uv[2] * uv[2];
+    const S d2v = vv[0] * vv[0] + vv[1] * vv[1] + vv[2] * vv[2];
+    const S vol = tv[2] * (uv[0] * vv[1] - vv[0] * uv[1]) - uv[2] * (tv[0] * vv[1] - vv[0] * tv[1]) +
+                  vv[2] * (tv[0] * uv[1] - uv[0] * tv[1]);
+    S w[3];
+    {
+        const S x0 = uv[1] * vv[2] - uv[2] * vv[1], x1 = uv[2] * vv[0] - uv[0] * vv[2],
+                x2 = uv[0] * vv[1] - uv[1] * vv[0];
+        w[0] = d2t * x0;
+        w[1] = d2t * x1;
+        w[2] = d2t * x2;
+    }
+    {
+        const S x0 = vv[1] * tv[2] - vv[2] * tv[1], x1 = vv[2] * tv[0] - vv[0] * tv[2],
+                x2 = vv[0] * tv[1] - vv[1] * tv[0];
+        w[0] += d2u * x0;
+        w[1] += d2u * x1;
+        w[2] += d2u * x2;
+    }
+    {
+        const S x0 = tv[1] * uv[2] - tv[2] * uv[1], x1 = tv[2] * uv[0] - tv[0] * uv[2],
+                x2 = tv[0] * uv[1] - tv[1] * uv[0];
+        w[0] += d2v * x0;
+        w[1] += d2v * x1;
+        w[2] += d2v * x2;
+    }
+    const S wn = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
+    const S rc = wn / ((S)4 * vol * vol);
+    *own = tid == i1;
+    return rc <= qa.r * qa.r && rc <= qb.r * qb.r && rc <= qc.r * qc.r && rc <= qd.r * qd.r;
+}
+
+// Outputs of a node with fewer than three candidates.
+template <class S> __device__ __forceinline__ void empty_star(const Ash3Args<S>& a, uint32_t tid) {
+    a.node_is_bnd[tid] = 1;
+    a.nelem_out[tid] = 0;
+    a.nelem[tid] = 0;
+    a.nfneig[tid] = 0;
+}
+
+// Local Delaunay of node tid's star + alpha filter (cpp:380-682), one lane,
+// every undecided sign through the exact stage.
+template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, uint32_t tid, uint8_t* cyc, double* ws) {
     const uint32_t n = a.n;
     const Sph4<S>* P = a.P;
     const uint32_t ncand = a.nineig[tid];
-    const uint32_t lane = threadIdx.x & 63u;
     auto neig = [&](uint32_t j) -> uint32_t { return j < kNInf3D ? n + j : a.cand[slab3(tid, j - kNInf3D, kCand3D)]; };
     auto T = [&](uint32_t ti) -> uint32_t& { return a.tet[slab3(tid, ti, kTet3D)]; };
-    auto C = [&](uint32_t v) -> uint8_t& { return cyc[v * 64u + lane]; };
+    auto C = [&](uint32_t v) -> uint8_t& { return cyc[v]; };
 
     T(0) = pack_tet(0, 2, 1);
     T(1) = pack_tet(1, 2, 3);
     T(2) = pack_tet(0, 1, 3);
     T(3) = pack_tet(0, 3, 2);
-    if (ncand - kNInf3D < 3) {
-        for (uint32_t j = 0; j + kNInf3D < ncand; ++j) a.active[slab3(tid, j, kCand3D)] = 0;
-        a.node_is_bnd[tid] = 1;
-        a.nelem_out[tid] = 0;
-        a.nelem[tid] = 0;
-        a.nfneig[tid] = 0;
-        return true;
-    }
     S pa0[3];
     load3(P, tid, pa0);
     uint32_t Tlast = 4;
@@ -192,234 +296,79 @@ __device__ bool local_delaunay3(const Ash3Args<S>& a, uint32_t tid, uint8_t* cyc
         S pe0[3];
         load3(P, curr, pe0);
         uint32_t Rsize = 0;
-        if constexpr (!EXACT) {
-            // Fast path (filters only; a node whose filter cannot decide is
-            // redone by the exact kernel, which takes the sequential loop below).
-            // Conflict flags of the current tetrahedra with the new point, bit
-            // k of word k >> 6 (f0..f3) for position k: every tetrahedron is
-            // tested once, two per step so that their loads overlap.
-            uint64_t f0 = 0, f1 = 0, f2 = 0, f3 = 0;
-            auto flag = [&](uint32_t k) -> bool {
-                const uint64_t w = k < 64 ? f0 : (k < 128 ? f1 : (k < 192 ? f2 : f3));
-                return (w >> (k & 63u)) & 1u;
-            };
-            auto set_flag = [&](uint32_t k, bool v) {
-                const uint64_t m = 1ull << (k & 63u);
-                const uint32_t q = k >> 6;
-                f0 = q == 0 ? (v ? f0 | m : f0 & ~m) : f0;
-                f1 = q == 1 ? (v ? f1 | m : f1 & ~m) : f1;
-                f2 = q == 2 ? (v ? f2 | m : f2 & ~m) : f2;
-                f3 = q == 3 ? (v ? f3 | m : f3 & ~m) : f3;
-            };
-            // first flagged position >= k (256 when none)
-            auto next_flag = [&](uint32_t k) -> uint32_t {
-#pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) {
-                    if (k < q * 64 + 64) {
-                        uint64_t m = q == 0 ? f0 : (q == 1 ? f1 : (q == 2 ? f2 : f3));
-                        if (k > q * 64) m &= ~0ull << (k - q * 64);
-                        if (m) return q * 64 + (uint32_t)__builtin_ctzll(m);
+        uint32_t ti = 0;
+        while (ti < Tlast) {
+            const uint32_t tl = T(ti);
+            const uint32_t la = tl & 255u, lb = (tl >> 8) & 255u, lc = (tl >> 16) & 255u;
+            uint32_t i2 = neig(la), i3 = neig(lb), i4 = neig(lc);
+            S pb[3], pc[3], pd[3];
+            load3(P, i2, pb);
+            load3(P, i3, pc);
+            load3(P, i4, pd);
+            S err;
+            S det = -insphere_filter(pa0, pb, pc, pd, pe0, &err);
+            if (!((det > err) || (-det > err))) {
+                uint32_t i1 = tid, i5 = curr;
+                S qa[3] = {pa0[0], pa0[1], pa0[2]}, qe[3] = {pe0[0], pe0[1], pe0[2]};
+                S* p1 = qa;
+                S* p2 = pb;
+                S* p3 = pc;
+                S* p4 = pd;
+                S* p5 = qe;
+                bool swap = false;
+                auto cs = [&](uint32_t& x, uint32_t& y, S*& px, S*& py) {
+                    if (x > y) {
+                        const uint32_t t = x;
+                        x = y;
+                        y = t;
+                        S* u = px;
+                        px = py;
+                        py = u;
+                        swap = !swap;
                     }
-                }
-                return 256u;
-            };
-            // point ids of the pair at t0 (the second repeats the first past
-            // the end); the next pair's ids load while the current pair is tested
-            auto pair_ids = [&](uint32_t t0, uint32_t (&o)[2][3]) {
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const uint32_t tl = T(u == 0 || t0 + 1 >= Tlast ? t0 : t0 + 1);
-                    o[u][0] = neig(tl & 255u);
-                    o[u][1] = neig((tl >> 8) & 255u);
-                    o[u][2] = neig((tl >> 16) & 255u);
-                }
-            };
-            uint32_t ids[2][3];
-            if (Tlast) pair_ids(0, ids);
-            for (uint32_t t0 = 0; t0 < Tlast; t0 += 2) {
-                const bool two = t0 + 1 < Tlast;
-                S pb[2][3], pc[2][3], pd[2][3];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    load3(P, ids[u][0], pb[u]);
-                    load3(P, ids[u][1], pc[u]);
-                    load3(P, ids[u][2], pd[u]);
-                }
-                uint32_t nids[2][3];
-                const bool more = t0 + 2 < Tlast;
-                if (more) pair_ids(t0 + 2, nids);
-                S det[2], err[2];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) det[u] = -insphere_filter(pa0, pb[u], pc[u], pd[u], pe0, &err[u]);
-                bool pos[2];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    pos[u] = det[u] > (S)0;
-                    if (u == 1 && !two) break;
-                    if ((det[u] > err[u]) || (-det[u] > err[u])) continue;
-                    if constexpr (sizeof(S) == sizeof(double)) {
-                        return false;
+                };
+                cs(i1, i5, p1, p5);
+                cs(i2, i4, p2, p4);
+                cs(i1, i3, p1, p3);
+                cs(i3, i5, p3, p5);
+                cs(i1, i2, p1, p2);
+                cs(i3, i4, p3, p4);
+                cs(i2, i5, p2, p5);
+                cs(i2, i3, p2, p3);
+                cs(i4, i5, p4, p5);
+                det = (S)-insphere_exact(p1, p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
+                int depth = 0;
+                while (det == (S)0) {
+                    ++depth;
+                    if (depth == 1) {
+                        bool c1;
+                        det = orient3d_filter(p2, p3, p4, p5, &c1);
+                        if (!c1) det = (S)orient3d_exact(p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
+                    } else if (depth == 2) {
+                        bool c2;
+                        det = orient3d_filter(p1, p3, p4, p5, &c2);
+                        if (!c2) det = (S)orient3d_exact(p1, p3, p4, p5, ws, (int)kExactWs3D, &over);
+                        det = -det;
                     } else {
-                        // FP32 inputs: the FP64 filter on the same (exactly
-                        // widened) coordinates certifies most of the signs the
-                        // FP32 filter cannot; the rest go to the exact kernel
-                        double qa[3], qb[3], qc[3], qd[3], qe[3];
-#pragma unroll
-                        for (int v = 0; v < 3; ++v) {
-                            qa[v] = pa0[v];
-                            qb[v] = pb[u][v];
-                            qc[v] = pc[u][v];
-                            qd[v] = pd[u][v];
-                            qe[v] = pe0[v];
-                        }
-                        double e2;
-                        const double d2 = -insphere_filter(qa, qb, qc, qd, qe, &e2);
-                        if (!((d2 > e2) || (-d2 > e2))) return false;
-                        pos[u] = d2 > 0.0;
+                        det = swap ? (S)1 : (S)-1;
                     }
                 }
-                if (pos[0]) set_flag(t0, true);
-                if (two && pos[1]) set_flag(t0 + 1, true);
-                if (more) {
-#pragma unroll
-                    for (int u = 0; u < 2; ++u)
-#pragma unroll
-                        for (int v = 0; v < 3; ++v) ids[u][v] = nids[u][v];
-                }
+                if (swap) det = -det;
             }
-            // The cavity: the sequential order of cpp:421-495 (a conflicting
-            // tetrahedron is swapped with the last one, which is tested next at
-            // the same position) replayed from the flags.
-            for (uint32_t ti = next_flag(0); ti < Tlast; ti = next_flag(ti)) {
+            if (det > (S)0) {
                 ++Rsize;
                 --Tlast;
-                const uint32_t tl = T(ti);
                 T(ti) = T(Tlast);
                 T(Tlast) = tl;
-                set_flag(ti, flag(Tlast));
-                set_flag(Tlast, true);
-            }
-        } else {
-            uint32_t ti = 0;
-            while (ti < Tlast) {
-                const uint32_t tl = T(ti);
-                const uint32_t la = tl & 255u, lb = (tl >> 8) & 255u, lc = (tl >> 16) & 255u;
-                uint32_t i2 = neig(la), i3 = neig(lb), i4 = neig(lc);
-                S pb[3], pc[3], pd[3];
-                load3(P, i2, pb);
-                load3(P, i3, pc);
-                load3(P, i4, pd);
-                S err;
-                S det = -insphere_filter(pa0, pb, pc, pd, pe0, &err);
-                if (!((det > err) || (-det > err))) {
-                    if constexpr (!EXACT) {
-                        return false;
-                    } else {
-                        uint32_t i1 = tid, i5 = curr;
-                        S qa[3] = {pa0[0], pa0[1], pa0[2]}, qe[3] = {pe0[0], pe0[1], pe0[2]};
-                        S* p1 = qa;
-                        S* p2 = pb;
-                        S* p3 = pc;
-                        S* p4 = pd;
-                        S* p5 = qe;
-                        bool swap = false;
-                        auto cs = [&](uint32_t& x, uint32_t& y, S*& px, S*& py) {
-                            if (x > y) {
-                                const uint32_t t = x;
-                                x = y;
-                                y = t;
-                                S* u = px;
-                                px = py;
-                                py = u;
-                                swap = !swap;
-                            }
-                        };
-                        cs(i1, i5, p1, p5);
-                        cs(i2, i4, p2, p4);
-                        cs(i1, i3, p1, p3);
-                        cs(i3, i5, p3, p5);
-                        cs(i1, i2, p1, p2);
-                        cs(i3, i4, p3, p4);
-                        cs(i2, i5, p2, p5);
-                        cs(i2, i3, p2, p3);
-                        cs(i4, i5, p4, p5);
-                        det = (S)-insphere_exact(p1, p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
-                        int depth = 0;
-                        while (det == (S)0) {
-                            ++depth;
-                            if (depth == 1) {
-                                bool c1;
-                                det = orient3d_filter(p2, p3, p4, p5, &c1);
-                                if (!c1) det = (S)orient3d_exact(p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
-                            } else if (depth == 2) {
-                                bool c2;
-                                det = orient3d_filter(p1, p3, p4, p5, &c2);
-                                if (!c2) det = (S)orient3d_exact(p1, p3, p4, p5, ws, (int)kExactWs3D, &over);
-                                det = -det;
-                            } else {
-                                det = swap ? (S)1 : (S)-1;
-                            }
-                        }
-                        if (swap) det = -det;
-                    }
-                }
-                if (det > (S)0) {
-                    ++Rsize;
-                    --Tlast;
-                    T(ti) = T(Tlast);
-                    T(Tlast) = tl;
-                } else {
-                    ++ti;
-                }
+            } else {
+                ++ti;
             }
         }
         if (Rsize) {
             // the star's tetrahedra use local ids below pi only
             for (uint32_t v = 0; v < pi; ++v) C(v) = (uint8_t)kEmpty;
-            --Rsize;
-            const uint32_t tlst = T(Tlast + Rsize);
-            const uint32_t ta = tlst & 255u, tb = (tlst >> 8) & 255u, tc3 = (tlst >> 16) & 255u;
-            C(ta) = (uint8_t)tb;
-            C(tb) = (uint8_t)tc3;
-            C(tc3) = (uint8_t)ta;
-            uint32_t cur = Tlast;
-            uint32_t first = ta;
-            int swap_with = (int)(Tlast + Rsize) - 1;
-            int niter = 0;
-            while (Rsize && niter++ < 100) {
-                const uint32_t tw = T(cur);
-                const uint32_t tcv[3] = {tw & 255u, (tw >> 8) & 255u, (tw >> 16) & 255u};
-                const uint32_t ty[3] = {C(tcv[0]), C(tcv[1]), C(tcv[2])};
-                bool inb[3], opp[3];
-#pragma unroll
-                for (int e = 0; e < 3; ++e) {
-                    inb[e] = ty[e] != kEmpty;
-                    opp[e] = ty[(e + 1) % 3] == tcv[e];
-                }
-                bool simple = opp[0] || opp[1] || opp[2];
-#pragma unroll
-                for (int e = 0; e < 3; ++e) simple &= (opp[e] || opp[(e + 1) % 3] || !inb[(e + 1) % 3]);
-                if (!simple) {
-                    ++cur;
-                    if ((int)cur > swap_with) cur = Tlast;
-                    continue;
-                }
-#pragma unroll
-                for (int e = 0; e < 3; ++e)
-                    if (!opp[e]) C(tcv[e]) = (uint8_t)tcv[(e + 1) % 3];
-#pragma unroll
-                for (int e = 0; e < 3; ++e) {
-                    if (opp[e] && opp[(e + 1) % 3]) {
-                        if (first == tcv[(e + 1) % 3]) first = ty[(e + 1) % 3];
-                        C(tcv[(e + 1) % 3]) = (uint8_t)kEmpty;
-                    }
-                }
-                T(cur) = T((uint32_t)swap_with);
-                T((uint32_t)swap_with) = tw;
-                --swap_with;
-                --Rsize;
-                cur = Tlast;
-            }
+            uint32_t first;
+            cavity_walk(T, C, Tlast, Rsize, &first);
             uint32_t c = first;
             int guard = 0;
             do {
@@ -442,66 +391,22 @@ __device__ bool local_delaunay3(const Ash3Args<S>& a, uint32_t tid, uint8_t* cyc
     while (ti < Tlast) {
         const uint32_t tl = T(ti);
         const uint32_t la = tl & 255u, lb = (tl >> 8) & 255u, lc = (tl >> 16) & 255u;
-        if (la < kNInf3D || lb < kNInf3D || lc < kNInf3D) {
+        bool own = false;
+        const bool inf = la < kNInf3D || lb < kNInf3D || lc < kNInf3D;
+        if (inf || !alpha_keep(P, tid, neig(la), neig(lb), neig(lc), &own)) {
             bnd = true;
             --Tlast;
             T(ti) = T(Tlast);
             continue;
         }
-        uint32_t i1 = tid, i2 = neig(la), i3 = neig(lb), i4 = neig(lc), t;
-        if (i1 > i3) { t = i3; i3 = i1; i1 = t; }
-        if (i2 > i4) { t = i4; i4 = i2; i2 = t; }
-        if (i1 > i2) { t = i2; i2 = i1; i1 = t; }
-        if (i3 > i4) { t = i4; i4 = i3; i3 = t; }
-        if (i2 > i3) { t = i3; i3 = i2; i2 = t; }
-        const Sph4<S> qa = P[i1], qb = P[i2], qc = P[i3], qd = P[i4];
-        const S tv[3] = {qa.c[0] - qd.c[0], qa.c[1] - qd.c[1], qa.c[2] - qd.c[2]};
-        const S uv[3] = {qb.c[0] - qd.c[0], qb.c[1] - qd.c[1], qb.c[2] - qd.c[2]};
-        const S vv[3] = {qc.c[0] - qd.c[0], qc.c[1] - qd.c[1], qc.c[2] - qd.c[2]};
-        const S d2t = tv[0] * tv[0] + tv[1] * tv[1] + tv[2] * tv[2];
-        const S d2u = uv[0] * uv[0] + uv[1] * uv[1] + uv[2] * uv[2];
-        const S d2v = vv[0] * vv[0] + vv[1] * vv[1] + vv[2] * vv[2];
-        const S vol = tv[2] * (uv[0] * vv[1] - vv[0] * uv[1]) - uv[2] * (tv[0] * vv[1] - vv[0] * tv[1]) +
-                      vv[2] * (tv[0] * uv[1] - uv[0] * tv[1]);
-        S w[3];
-        {
-            const S x0 = uv[1] * vv[2] - uv[2] * vv[1], x1 = uv[2] * vv[0] - uv[0] * vv[2],
-                    x2 = uv[0] * vv[1] - uv[1] * vv[0];
-            w[0] = d2t * x0;
-            w[1] = d2t * x1;
-            w[2] = d2t * x2;
-        }
-        {
-            const S x0 = vv[1] * tv[2] - vv[2] * tv[1], x1 = vv[2] * tv[0] - vv[0] * tv[2],
-                    x2 = vv[0] * tv[1] - vv[1] * tv[0];
-            w[0] += d2u * x0;
-            w[1] += d2u * x1;
-            w[2] += d2u * x2;
-        }
-        {
-            const S x0 = tv[1] * uv[2] - tv[2] * uv[1], x1 = tv[2] * uv[0] - tv[0] * uv[2],
-                    x2 = tv[0] * uv[1] - tv[1] * uv[0];
-            w[0] += d2v * x0;
-            w[1] += d2v * x1;
-            w[2] += d2v * x2;
-        }
-        const S wn = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
-        const S rc = wn / ((S)4 * vol * vol);
-        if (rc <= qa.r * qa.r && rc <= qb.r * qb.r && rc <= qc.r * qc.r && rc <= qd.r * qd.r) {
-            C(la) = (uint8_t)(C(la) + 1);
-            C(lb) = (uint8_t)(C(lb) + 1);
-            C(lc) = (uint8_t)(C(lc) + 1);
-            ++nloc;
-            if (tid == i1) {
-                ++nout;
-                ++ti;
-            } else {
-                --Tlast;
-                T(ti) = T(Tlast);
-                T(Tlast) = tl;
-            }
+        C(la) = (uint8_t)(C(la) + 1);
+        C(lb) = (uint8_t)(C(lb) + 1);
+        C(lc) = (uint8_t)(C(lc) + 1);
+        ++nloc;
+        if (own) {
+            ++nout;
+            ++ti;
         } else {
-            bnd = true;
             --Tlast;
             T(ti) = T(Tlast);
         }
@@ -518,21 +423,642 @@ __device__ bool local_delaunay3(const Ash3Args<S>& a, uint32_t tid, uint8_t* cyc
     a.nelem_out[tid] = (uint8_t)nout;
     a.nelem[tid] = (uint8_t)nloc;
     a.nfneig[tid] = nf;
-    return true;
 }
 
-// Four wavefronts per block (one LDS cycle buffer each), one node per lane.
-// Lanes keep consecutive (Morton-ordered) nodes: neighbouring nodes share
-// most candidates, so their coordinate loads hit the same cache lines.
-constexpr uint32_t kDelaunay3Block = 256;
-template <class S> __global__ __launch_bounds__(kDelaunay3Block) void delaunay3_kernel(Ash3Args<S> a) {
-    __shared__ uint8_t cyc[kDelaunay3Block / 64][kCycle3D * 64];
-    const uint32_t tid = blockIdx.x * kDelaunay3Block + threadIdx.x;
-    if (tid >= a.n) return;
-    if (!local_delaunay3<S, false>(a, tid, cyc[threadIdx.x >> 6], nullptr)) {
-        const uint32_t k = atomicAdd(&a.queue[0], 1u);
-        a.queue[2 + k] = tid;
+// Local Delaunay + alpha filter of every node, 16 lanes per node.
+//
+// A star holds about 23 tetrahedra while 34 to 80 candidates go in, two of
+// three of which open a cavity of about 5.  One lane per node spent its time
+// gathering three corners for each of the ~1,500 insphere tests of a node (a
+// cache line per lane and load).  Here 16 lanes hold the star: lane l the
+// tetrahedra at positions l, l + 16, ... in registers, the ids also in LDS.
+//
+//   test    With the node as origin, corners b, c, d and the new point e, the
+//           insphere value is e.W - V |e|^2 with W = |b|^2 cxd + |c|^2 dxb +
+//           |d|^2 bxc and V = b.(cxd).  W, V and the factors wp, vp of the
+//           error bound are kept per tetrahedron, so a test is 7 FP32
+//           operations on one LDS read.  Coordinates are relative to the
+//           node, divided by a power of two near alpha and rounded to FP32 in
+//           both node types.  Each monomial sees at most 21 roundings and the
+//           bound takes 24 (kSphBound); the sums of absolute monomials are
+//           bounded by the lengths: a component of |c||x||d| by |c| |d|, so
+//           W's by Q (|b| + |c| + |d|) and V's by sqrt(3) Q, Q = |b| |c| |d|.
+//           kSphFloor covers underflow for coordinates up to kSphRange,
+//           beyond which the point is NaN and certifies nothing.  What FP32
+//           cannot certify goes to the FP64 filter on the node's own
+//           coordinates, and a node where that fails too to the exact kernel.
+//           A certified sign is the exact sign, so all three give the same
+//           decisions.
+//   remove  The sequential swap with the last (cpp:421-495) fills the flagged
+//           positions below m (the number kept), in order, with the kept ones
+//           from the end backwards.  With j flagged positions below p, a
+//           flagged p takes the j-th of these, and a kept p >= m is the
+//           (m - 1 - p + j)-th.  The removed ones end up from m on: the
+//           flagged one at q > m at q - 1, the j-th other one right below
+//           where the (j-1)-th moved one came from.
+//   cycle   One removed triangle per lane, a set of lanes per corner: the
+//           lanes that hold both ends of an edge are its two triangles, so an
+//           edge whose other triangle stays is on the boundary cycle.  The
+//           reference's walk ends on the same cycle, and starts there from the
+//           first removed triangle's first corner, unless that corner ends
+//           inside: then the start is, as often as needed, the corner before
+//           it in the triangle that closes the fan around it.  Which one that
+//           is depends on the order of the walk, so the walk runs, on sets of
+//           lanes: a triangle can join the disc when it shares two edges with
+//           it, or one and the third corner is not in it yet, and the scan
+//           takes the one at the lowest position, after one failed step per
+//           position before.  A cavity of 14 or fewer is done in at most 91
+//           steps (at most one fails per remaining triangle), so the cap of
+//           100 plays no part.  One of up to 32 has two triangles per lane;
+//           where its walk meets the cap, in larger ones and in stars that the
+//           cap left open, the reference's own walk runs.
+//   new     One lane per new tetrahedron computes its W, V and bounds; the
+//           lane that holds the position picks them up through LDS.
+//
+// A star that outgrows 64 positions goes to the exact kernel (queue[2] counts
+// these).
+//
+// Bound: instruction issue (364 vector and 264 scalar instructions per
+// insertion of a wavefront's four nodes, three quarters of the vector issue
+// slots at 4 wavefronts per SIMD).  5 wavefronts (96 registers) spill and are
+// a third slower.  From one lane per node to this: 1,996,920 FP64 nodes 68.7 ->
+// 26.5 ms, 100,000 FP32 ones 2.50 -> 0.69 ms, 20,102 FP32 ones (79 blocks of
+// one lane per node left most of the chip idle) 3.96 -> 0.49 ms.
+constexpr int kStarLanes = 16;
+constexpr uint32_t kStarTets = 64;
+constexpr int kStarSlots = (int)kStarTets / kStarLanes;
+constexpr float kSphBound = 1.7320509f * 24.0f * 5.9604644775390625e-08f;
+constexpr float kSphFloor = 1e-20f;
+constexpr float kSphRange = 1e7f;
+constexpr uint32_t kWalkFree = 14;  // R (R - 1) / 2 <= 100, and R + 2 new ones on 16 lanes
+
+// Candidates of the four nodes of a wavefront together (LDS); a node that does
+// not fit beside the others waits for a second pass.  34 to 85 candidates per
+// node are usual; 448 bring a wavefront's LDS to 10 KB, four per SIMD.
+constexpr uint32_t kStarPool = 448;
+
+struct SphReg {
+    float wx, wy, wz, v, wp, vp;
+    uint32_t w;  // ids (pack_tet)
+};
+struct alignas(16) SphRec {
+    SphReg r;
+    uint32_t pos;  // where it comes from
+};
+struct Star3Lds {
+    union {
+        uint32_t c[kCycle3D];    // per local id: set of lanes, next on the cycle, count
+        SphRec rec[kStarLanes];  // tetrahedra on their way to another lane
+    };
+    uint32_t t[kStarTets];  // ids: removed ones; the whole star for a large cavity
+};
+
+// LDS written by other lanes of this wavefront: program order is execution
+// order there, so only the compiler has to be held.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ uint64_t ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+// Bits of this lane's group of 16 in a wavefront ballot.
+__device__ __forceinline__ uint32_t group_bits(uint64_t m, uint32_t grp) {
+    const uint32_t h = grp >= 2 ? (uint32_t)(m >> 32) : (uint32_t)m;
+    return (h >> ((grp & 1u) * 16u)) & 0xffffu;
+}
+// Two ballots' bits of this lane's group, the second one's in the upper half.
+__device__ __forceinline__ uint32_t group_bits2(uint64_t m0, uint64_t m1, uint32_t grp) {
+    const uint32_t h0 = grp >= 2 ? (uint32_t)(m0 >> 32) : (uint32_t)m0;
+    const uint32_t h1 = grp >= 2 ? (uint32_t)(m1 >> 32) : (uint32_t)m1;
+    return __builtin_amdgcn_perm(h1, h0, (grp & 1u) ? 0x07060302u : 0x05040100u);
+}
+// Minimum over the 16 lanes of the group (a DPP row).
+__device__ __forceinline__ uint32_t group_min(uint32_t v) {
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x128, 0xf, 0xf, false));  // row_ror:8
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x124, 0xf, 0xf, false));  // row_ror:4
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x122, 0xf, 0xf, false));  // row_ror:2
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x121, 0xf, 0xf, false));  // row_ror:1
+    return v;
+}
+// A set of up to 64 positions.
+struct PosSet {
+    uint32_t lo, hi;
+};
+
+// The FP64 filter's sign of the insphere test of e against the tetrahedron
+// (a, b, c, d): 1 inside, -1 outside, 0 undecided.
+template <class S>
+__device__ __forceinline__ int insphere_side_f64(const Sph4<S>* P, uint32_t ia, uint32_t ib, uint32_t ic, uint32_t id,
+                                              uint32_t ie) {
+    const Sph4<S> q[5] = {P[ia], P[ib], P[ic], P[id], P[ie]};
+    double x[5][3];
+#pragma unroll
+    for (int v = 0; v < 5; ++v)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) x[v][k] = q[v].c[k];
+    double err;
+    const double det = -insphere_filter(x[0], x[1], x[2], x[3], x[4], &err);
+    return det > err ? 1 : (-det > err ? -1 : 0);
+}
+
+template <class S>
+__device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, uint32_t ncand, uint32_t sub,
+                                           uint32_t grp, float4* E, Star3Lds& L) {
+    constexpr int G = kStarLanes, NS = kStarSlots;
+    const uint32_t n = a.n;
+    const Sph4<S>* P = a.P;
+    auto neig = [&](uint32_t j) -> uint32_t { return j < kNInf3D ? n + j : a.cand[slab3(tid, j - kNInf3D, kCand3D)]; };
+    const Sph4<S> self = P[tid];
+    {
+        const double r = (double)self.r;
+        const double scale = (r > 0.0 && r < 1e300) ? ldexp(1.0, -ilogb(r)) : 1.0;
+        for (uint32_t j = sub; j < ncand; j += G) {
+            const Sph4<S> q = P[neig(j)];
+            float4 e;
+            e.x = (float)(((double)q.c[0] - (double)self.c[0]) * scale);
+            e.y = (float)(((double)q.c[1] - (double)self.c[1]) * scale);
+            e.z = (float)(((double)q.c[2] - (double)self.c[2]) * scale);
+            if (!(fmaxf(fabsf(e.x), fmaxf(fabsf(e.y), fabsf(e.z))) <= kSphRange)) e.x = NAN;
+            e.w = sqrtf(fmaf(e.x, e.x, fmaf(e.y, e.y, e.z * e.z)));
+            E[j] = e;
+        }
     }
+    wave_lds_sync();
+    uint32_t Tl = 4;
+    SphReg rec[NS];
+    // corners b, c, d (ids w); |c|^2 dxb + |d|^2 bxc = b x (|d|^2 c - |c|^2 d)
+    auto make_rec = [&](uint32_t w, const float4& b, const float4& c, const float4& d) {
+        const float x = fmaf(c.y, d.z, -(c.z * d.y)), y = fmaf(c.z, d.x, -(c.x * d.z)),
+                    z = fmaf(c.x, d.y, -(c.y * d.x));
+        const float bb = b.w * b.w, cc = c.w * c.w, dd = d.w * d.w;
+        const float gx = fmaf(dd, c.x, -(cc * d.x)), gy = fmaf(dd, c.y, -(cc * d.y)), gz = fmaf(dd, c.z, -(cc * d.z));
+        const float q = kSphBound * (b.w * c.w) * d.w;
+        SphReg r;
+        r.wx = fmaf(bb, x, fmaf(b.y, gz, -(b.z * gy)));
+        r.wy = fmaf(bb, y, fmaf(b.z, gx, -(b.x * gz)));
+        r.wz = fmaf(bb, z, fmaf(b.x, gy, -(b.y * gx)));
+        r.v = fmaf(b.x, x, fmaf(b.y, y, b.z * z));
+        // sum |e_k| <= sqrt(3) |e|
+        r.wp = q * (b.w + c.w + d.w);
+        r.vp = q;
+        r.w = w;
+        return r;
+    };
+    auto load_rec = [&](uint32_t w) { return make_rec(w, E[w & 255u], E[(w >> 8) & 255u], E[(w >> 16) & 255u]); };
+    if (sub < 4) {
+        const uint32_t w = sub == 0   ? pack_tet(0, 2, 1)
+                           : sub == 1 ? pack_tet(1, 2, 3)
+                           : sub == 2 ? pack_tet(0, 1, 3)
+                                      : pack_tet(0, 3, 2);
+        rec[0] = load_rec(w);
+    }
+    const uint32_t below[2] = {(1u << sub) - 1u, (1u << (sub + 16)) - 1u};
+    auto has = [&](const PosSet& F, int s) -> bool { return ((s < 2 ? F.lo : F.hi) >> ((s & 1) * 16 + sub)) & 1u; };
+    auto rank = [&](const PosSet& F, int s) -> uint32_t {  // members of F below this lane's position in slot s
+        return s < 2 ? __popc(F.lo & below[s & 1]) : __popc(F.hi & below[s & 1]) + __popc(F.lo);
+    };
+    auto members = [](const PosSet& F) -> uint32_t { return __popc(F.lo) + __popc(F.hi); };
+    auto word = [&](uint32_t s) -> uint32_t {
+        return s == 0 ? rec[0].w : (s == 1 ? rec[1].w : (s == 2 ? rec[2].w : rec[3].w));
+    };
+    bool open_star = false;
+    uint32_t redo = 0;  // 1: undecided sign, 2: too many tetrahedra or a broken cycle
+    for (uint32_t pi = kNInf3D; pi < ncand; ++pi) {
+        const float4 e = E[pi];
+        const float ee = e.w * e.w;
+        // lane constants are cheaper to form again than to hold
+        asm volatile("" : "+v"(sub));
+        const bool wide = ballot(Tl > 32) != 0;  // some node of the wavefront uses slots 2 and 3
+        uint64_t in_m[NS];
+        bool un[NS];
+        auto test = [&](int s) {
+            const SphReg& r = rec[s];
+            const float det = fmaf(e.x, r.wx, fmaf(e.y, r.wy, fmaf(e.z, r.wz, -(ee * r.v))));
+            const float err = fmaf(r.wp, e.w, fmaf(r.vp, ee, kSphFloor));
+            const bool in = (uint32_t)(s * G) + sub < Tl;
+            in_m[s] = ballot(in && det > err);
+            un[s] = in && !(fabsf(det) > err);
+        };
+        test(0);
+        test(1);
+        PosSet F;
+        F.lo = group_bits2(in_m[0], in_m[1], grp);
+        F.hi = 0;
+        uint64_t un_m = ballot(un[0] || un[1]);
+        un[2] = un[3] = false;
+        if (wide) {
+            test(2);
+            test(3);
+            F.hi = group_bits2(in_m[2], in_m[3], grp);
+            un_m |= ballot(un[2] || un[3]);
+        }
+        if (__builtin_expect(un_m != 0, 0)) {
+            const uint32_t unsure = un[0] | (un[1] << 1) | (un[2] << 2) | (un[3] << 3);
+            bool undecided = false;
+            // the FP64 test needs the records' registers
+            volatile SphReg save[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                save[s].wx = rec[s].wx;
+                save[s].wy = rec[s].wy;
+                save[s].wz = rec[s].wz;
+                save[s].v = rec[s].v;
+                save[s].wp = rec[s].wp;
+                save[s].vp = rec[s].vp;
+                save[s].w = rec[s].w;
+            }
+#pragma unroll 1
+            for (uint32_t k = 0; k < (uint32_t)NS; ++k) {
+                bool pos = false;
+                if ((unsure >> k) & 1u) {
+                    const uint32_t tw = save[k].w;
+                    const int side = insphere_side_f64(P, tid, neig(tw & 255u), neig((tw >> 8) & 255u),
+                                                       neig((tw >> 16) & 255u), neig(pi));
+                    pos = side > 0;
+                    undecided |= side == 0;
+                }
+                const uint32_t bits = group_bits(ballot(pos), grp) << ((k & 1u) * 16u);
+                F.lo |= k < 2 ? bits : 0u;
+                F.hi |= k < 2 ? 0u : bits;
+            }
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                rec[s].wx = save[s].wx;
+                rec[s].wy = save[s].wy;
+                rec[s].wz = save[s].wz;
+                rec[s].v = save[s].v;
+                rec[s].wp = save[s].wp;
+                rec[s].vp = save[s].vp;
+                rec[s].w = save[s].w;
+            }
+            if (group_bits(ballot(undecided), grp)) {
+                redo = 1;
+                break;
+            }
+        }
+        const uint32_t R = members(F);
+        if (R == 0) continue;
+        const uint32_t m = Tl - R;
+        uint32_t end = m;
+        if (__builtin_expect(R <= kWalkFree && !open_star, 1)) {
+            // moved and removed tetrahedra
+            auto move_out = [&](int s) {
+                const uint32_t p = (uint32_t)(s * G) + sub;
+                if (p >= m && p < Tl && !has(F, s)) L.rec[m - 1 - p + rank(F, s)] = SphRec{rec[s], p};
+            };
+            auto move_in = [&](int s) {
+                const uint32_t p = (uint32_t)(s * G) + sub;
+                if (has(F, s)) {
+                    const uint32_t j = rank(F, s), w = rec[s].w;
+                    const uint32_t at = p > m ? p : (j ? L.rec[j - 1].pos : Tl);
+                    L.t[at - 1 - m] = w;
+                    if (p < m) rec[s] = L.rec[j].r;
+                }
+            };
+            move_out(0);
+            move_out(1);
+            if (wide) {
+                move_out(2);
+                move_out(3);
+            }
+            wave_lds_sync();
+            move_in(0);
+            move_in(1);
+            if (wide) {
+                move_in(2);
+                move_in(3);
+            }
+            wave_lds_sync();
+            const uint32_t tw = L.t[sub], ta = L.t[R - 1] & 255u;  // (lanes from R on: any valid or stale ids)
+            const uint32_t x = tw & 127u, y = (tw >> 8) & 127u, z = (tw >> 16) & 127u;
+            if (sub < R) {
+                L.c[x] = 0;
+                L.c[y] = 0;
+                L.c[z] = 0;
+            }
+            wave_lds_sync();
+            if (sub < R) {
+                atomicOr(&L.c[x], 1u << sub);
+                atomicOr(&L.c[y], 1u << sub);
+                atomicOr(&L.c[z], 1u << sub);
+            }
+            wave_lds_sync();
+            uint32_t first = ta;
+            const uint32_t mx = L.c[x], my = L.c[y], mz = L.c[z], others = ~(1u << sub);
+            const uint32_t n0 = mx & my & others, n1 = my & mz & others, n2 = mz & mx & others;
+            const bool b0 = sub < R && n0 == 0, b1 = sub < R && n1 == 0, b2 = sub < R && n2 == 0;
+            auto on_cycle = [&](uint32_t v) -> bool {
+                return group_bits(ballot((b0 && x == v) || (b1 && y == v) || (b2 && z == v)), grp) != 0;
+            };
+            if (!on_cycle(first)) {
+                uint32_t disc = 1u << (R - 1), fan = L.c[first], left = R - 1;
+                uint32_t key = sub < R - 1 ? sub << 4 | sub : ~0u;  // position and lane; ~0: in the disc
+                while (left) {
+                    const bool o0 = n0 & disc, o1 = n1 & disc, o2 = n2 & disc;
+                    const bool joins = (o0 && (o1 || o2 || !(mz & disc))) || (o1 && (o2 || !(mx & disc))) ||
+                                       (o2 && !(my & disc));
+                    const uint32_t best = group_min(joins ? key : ~0u);
+                    if (best == ~0u) break;
+                    const uint32_t win = best & 15u;
+                    disc |= 1u << win;
+                    --left;
+                    // the last position's triangle takes the winner's
+                    key = key >> 4 == left ? (best & ~15u) | sub : key;
+                    key = sub == win ? ~0u : key;
+                    if ((fan & ~disc) == 0) {
+                        const uint32_t before = x == first ? z : (y == first ? x : y);
+                        first = (uint32_t)__shfl((int)before, (int)(grp * G + win), 64);
+                        if (on_cycle(first)) break;
+                        fan = L.c[first];
+                    }
+                }
+            }
+            wave_lds_sync();
+            if (b0) L.c[x] = y;
+            if (b1) L.c[y] = z;
+            if (b2) L.c[z] = x;
+            wave_lds_sync();
+            // around the cycle (and on, until the wavefront's longest one is
+            // closed); lane b keeps the start of the b-th edge
+            uint32_t c = first, mc = first;
+            uint64_t open_m = ballot(true);
+            for (uint32_t k = 1; k < (uint32_t)G && open_m; ++k) {
+                c = L.c[c & (kCycle3D - 1)];
+                mc = sub == k ? c : mc;
+                open_m &= ballot(c != first);
+            }
+            const uint32_t mn = L.c[mc & (kCycle3D - 1)];
+            const uint32_t again = group_bits(ballot(sub != 0 && mc == first), grp) & ~1u;
+            const uint32_t nb = again ? (uint32_t)__builtin_ctz(again) : (uint32_t)G;
+            end = m + nb;
+            // (a proper boundary has R + 2 edges, less two per corner inside)
+            if (group_bits(ballot(sub + 1 == nb && mn != first), grp) || nb > R + 2 || ((nb ^ R) & 1u) ||
+                end > kStarTets) {
+                redo = 2;
+                break;
+            }
+            wave_lds_sync();
+            if (sub < nb) L.rec[sub] = SphRec{make_rec(pack_tet(pi, mc, mn), e, E[mc], E[mn]), 0};
+            wave_lds_sync();
+            auto take = [&](int s) {
+                const uint32_t p = (uint32_t)(s * G) + sub;
+                if (p >= m && p < end) rec[s] = L.rec[p - m].r;
+            };
+            take(0);
+            take(1);
+            if (ballot(end > 32)) {
+                take(2);
+                take(3);
+            }
+            wave_lds_sync();
+        } else {
+            auto T = [&](uint32_t k) -> uint32_t& { return L.t[k]; };
+            auto C = [&](uint32_t k) -> uint32_t& { return L.c[k]; };
+            // as above for the ids alone; L.t becomes the whole star, the
+            // removed ones from m on
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const uint32_t p = (uint32_t)(s * G) + sub;
+                if (p >= m && p < Tl && !has(F, s)) L.c[m - 1 - p + rank(F, s)] = rec[s].w | p << 24;
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const uint32_t p = (uint32_t)(s * G) + sub;
+                if (has(F, s)) {
+                    const uint32_t j = rank(F, s);
+                    const uint32_t at = p > m ? p : (j ? L.c[j - 1] >> 24 : Tl);
+                    T(at - 1) = rec[s].w;
+                    if (p < m) T(p) = L.c[j] & 0xffffffu;
+                } else if (p < m) {
+                    T(p) = rec[s].w;
+                }
+            }
+            wave_lds_sync();
+            // every lane of the group runs what follows on the same words
+            uint32_t first = T(Tl - 1) & 255u;
+            bool walk = open_star || R > 2 * (uint32_t)G;
+            if (!walk) {
+                // as above with two triangles per lane, at sub and sub + 16
+                uint32_t x[2], y[2], z[2], n0[2], n1[2], n2[2], mx[2], my[2], mz[2], key[2];
+                bool b0[2], b1[2], b2[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t i = sub + h * G, tw = i < R ? T(m + i) : 0u;
+                    x[h] = tw & 255u;
+                    y[h] = (tw >> 8) & 255u;
+                    z[h] = (tw >> 16) & 255u;
+                    if (i < R) {
+                        C(x[h]) = 0;
+                        C(y[h]) = 0;
+                        C(z[h]) = 0;
+                    }
+                }
+                wave_lds_sync();
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t i = sub + h * G;
+                    if (i < R) {
+                        atomicOr(&C(x[h]), 1u << i);
+                        atomicOr(&C(y[h]), 1u << i);
+                        atomicOr(&C(z[h]), 1u << i);
+                    }
+                }
+                wave_lds_sync();
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t i = sub + h * G, others = ~(1u << i);
+                    mx[h] = C(x[h]);
+                    my[h] = C(y[h]);
+                    mz[h] = C(z[h]);
+                    n0[h] = mx[h] & my[h] & others;
+                    n1[h] = my[h] & mz[h] & others;
+                    n2[h] = mz[h] & mx[h] & others;
+                    b0[h] = i < R && n0[h] == 0;
+                    b1[h] = i < R && n1[h] == 0;
+                    b2[h] = i < R && n2[h] == 0;
+                    key[h] = i < R - 1 ? i << 5 | i : ~0u;
+                }
+                auto on_cycle = [&](uint32_t v) -> bool {
+                    bool on = false;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) on |= (b0[h] && x[h] == v) || (b1[h] && y[h] == v) || (b2[h] && z[h] == v);
+                    return group_bits(ballot(on), grp) != 0;
+                };
+                uint32_t disc = 1u << (R - 1), left = R - 1, steps = 0;
+                while (left) {
+                    uint32_t k = ~0u;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const bool o0 = n0[h] & disc, o1 = n1[h] & disc, o2 = n2[h] & disc;
+                        const bool joins = (o0 && (o1 || o2 || !(mz[h] & disc))) || (o1 && (o2 || !(mx[h] & disc))) ||
+                                           (o2 && !(my[h] & disc));
+                        k = joins ? min(k, key[h]) : k;
+                    }
+                    const uint32_t best = group_min(k);
+                    steps += (best >> 5) + 1;
+                    if (best == ~0u || steps > 100) break;
+                    const uint32_t win = best & 31u;
+                    disc |= 1u << win;
+                    --left;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        key[h] = key[h] >> 5 == left ? (best & ~31u) | (sub + h * G) : key[h];
+                        key[h] = sub + h * G == win ? ~0u : key[h];
+                    }
+                    if (!on_cycle(first) && (C(first) & ~disc) == 0) {
+                        const bool up = win >= (uint32_t)G;
+                        const uint32_t vx = up ? x[1] : x[0], vy = up ? y[1] : y[0], vz = up ? z[1] : z[0];
+                        const uint32_t before = vx == first ? vz : (vy == first ? vx : vy);
+                        first = (uint32_t)__shfl((int)before, (int)(grp * G + (win & 15u)), 64);
+                    }
+                }
+                walk = left != 0;
+                wave_lds_sync();
+                if (!walk) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        if (b0[h]) C(x[h]) = y[h];
+                        if (b1[h]) C(y[h]) = z[h];
+                        if (b2[h]) C(z[h]) = x[h];
+                    }
+                }
+            }
+            if (walk) {
+                for (uint32_t v = sub; v < kCycle3D; v += G) C(v) = kEmpty;
+                wave_lds_sync();
+                open_star |= cavity_walk(T, C, m, R, &first);
+            }
+            wave_lds_sync();
+            uint32_t c = first;
+            do {
+                if (c >= kCycle3D || end >= kStarTets) {
+                    redo = 2;
+                    break;
+                }
+                const uint32_t nx = C(c);
+                T(end++) = pack_tet(pi, c, nx);
+                c = nx;
+            } while (c != first);
+            if (redo) break;
+            wave_lds_sync();
+#pragma unroll 1
+            for (uint32_t k = 0; k * G < end; ++k) {
+                const uint32_t p = k * G + sub;
+                if (p < end) {
+                    const SphReg r = load_rec(T(p));
+                    if (k == 0) rec[0] = r;
+                    if (k == 1) rec[1] = r;
+                    if (k == 2) rec[2] = r;
+                    if (k == 3) rec[3] = r;
+                }
+            }
+            wave_lds_sync();
+        }
+        Tl = end;
+    }
+    if (redo) {
+        if (sub == 0) {
+            a.queue[kQueueIds + atomicAdd(&a.queue[0], 1u)] = tid;
+            if (redo == 2) atomicAdd(&a.queue[2], 1u);
+        }
+        return;
+    }
+    // alpha filter: kept tetrahedra count at their corners; this node's own
+    // ones come first, in the order the sequential filter leaves them in
+    for (uint32_t v = sub; v < ncand; v += G) L.c[v] = 0;
+    wave_lds_sync();
+    uint64_t own_m = 0;
+    uint32_t nloc = 0;
+#pragma unroll 1
+    for (uint32_t p0 = 0; p0 < Tl; p0 += G) {
+        const uint32_t p = p0 + sub;
+        bool keep = false, own = false;
+        if (p < Tl) {
+            const uint32_t tw = word(p0 / G);
+            const uint32_t la = tw & 255u, lb = (tw >> 8) & 255u, lc = (tw >> 16) & 255u;
+            if (la >= kNInf3D && lb >= kNInf3D && lc >= kNInf3D)
+                keep = alpha_keep(P, tid, neig(la), neig(lb), neig(lc), &own);
+            if (keep) {
+                atomicAdd(&L.c[la], 1u);
+                atomicAdd(&L.c[lb], 1u);
+                atomicAdd(&L.c[lc], 1u);
+            }
+        }
+        nloc += __popc(group_bits(ballot(keep), grp));
+        own_m |= (uint64_t)group_bits(ballot(keep && own), grp) << p0;
+    }
+    const uint32_t nout = __popcll(own_m);
+#pragma unroll 1
+    for (uint32_t p0 = 0; p0 < Tl; p0 += G) {
+        const uint32_t p = p0 + sub;
+        if (!((own_m >> p) & 1u)) continue;
+        // below nout they stay; the others fill the gaps from the end
+        uint32_t q = p;
+        if (p >= nout) {
+            uint32_t k = __popcll(own_m >> p) - 1;
+            uint64_t gaps = ~own_m;
+            while (k--) gaps &= gaps - 1;
+            q = __builtin_ctzll(gaps);
+        }
+        a.tet[slab3(tid, q, kTet3D)] = word(p0 / G);
+    }
+    uint32_t nf = 0;
+    for (uint32_t v0 = kNInf3D; v0 < ncand; v0 += G) {
+        const uint32_t v = v0 + sub;
+        const uint32_t c = v < ncand ? L.c[v] : 0u;
+        if (v < ncand) a.active[slab3(tid, v - kNInf3D, kCand3D)] = (uint8_t)c;
+        nf += __popc(group_bits(ballot(c != 0), grp));
+    }
+    if (sub == 0) {
+        a.node_is_bnd[tid] = nloc != Tl;
+        a.nelem_out[tid] = (uint8_t)nout;
+        a.nelem[tid] = (uint8_t)nloc;
+        a.nfneig[tid] = nf;
+    }
+}
+
+
+template <class S>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void star3_kernel(
+    Ash3Args<S> a, uint32_t blocks_per_xcd) {
+    constexpr uint32_t G = kStarLanes;
+    constexpr uint32_t NPW = 64 / G;
+    __shared__ float4 pool[kStarPool];
+    __shared__ Star3Lds lds[NPW];
+    const uint32_t sub = threadIdx.x % G, grp = threadIdx.x / G;
+    // consecutive nodes share candidates and slab lines: one XCD (blocks go to
+    // the XCDs in turn) takes a contiguous range of them
+    const uint32_t blk = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
+    const uint32_t tid = blk * NPW + grp;
+    const uint32_t n = a.n;
+    const uint32_t ncand = tid < n ? a.nineig[tid] : 0u;
+    if (tid < n && ncand - kNInf3D < 3) {
+        if (sub < ncand - kNInf3D) a.active[slab3(tid, sub, kCand3D)] = 0;
+        if (sub == 0) empty_star(a, tid);
+    }
+    // share of the pool: the nodes that fit, in order; the first one always does
+    uint32_t want = tid < n && ncand - kNInf3D >= 3 ? ncand : 0u;
+    while (ballot(want != 0)) {
+        uint32_t off = 0, mine = ~0u;
+#pragma unroll
+        for (uint32_t g = 0; g < NPW; ++g) {
+            const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)want, (int)(g * G));
+            if (k && off + k <= kStarPool) {
+                if (grp == g) mine = off;
+                off += k;
+            }
+        }
+        if (mine != ~0u) {
+            star3_node<S>(a, tid, ncand, sub, grp, pool + mine, lds[grp]);
+            want = 0;
+        }
+        wave_lds_sync();
+    }
+}
+
+template <class S> void launch_star3(const Ash3Args<S>& a, hipStream_t s) {
+    const uint32_t blocks = (a.n + 64 / kStarLanes - 1) / (64 / kStarLanes), per_xcd = (blocks + 7) / 8;
+    hipLaunchKernelGGL((star3_kernel<S>), dim3(8 * per_xcd), dim3(64), 0, s, a, per_xcd);
 }
 
 // One queued node per wavefront (lane 0; the block is one wavefront): the
@@ -540,11 +1066,11 @@ template <class S> __global__ __launch_bounds__(kDelaunay3Block) void delaunay3_
 // insertions, so nodes sharing a wavefront would run their exact stages one
 // after another.  The expansion workspace lives in LDS.
 template <class S> __global__ __launch_bounds__(64) void delaunay3_exact_kernel(Ash3Args<S> a) {
-    __shared__ uint8_t cyc[kCycle3D * 64];
+    __shared__ uint8_t cyc[kCycle3D];
     __shared__ double ws[kExactWs3D];
     if (threadIdx.x != 0) return;
     const uint32_t cnt = a.queue[0];
-    for (uint32_t k = blockIdx.x; k < cnt; k += gridDim.x) local_delaunay3<S, true>(a, a.queue[2 + k], cyc, ws);
+    for (uint32_t k = blockIdx.x; k < cnt; k += gridDim.x) local_delaunay3_exact<S>(a, a.queue[kQueueIds + k], cyc, ws);
 }
 
 // Slab -> CSR (cpp:692-735): edges with count <= 3 are boundary edges; the
@@ -634,7 +1160,7 @@ template <class S> void Ash3D<S>::init(hipStream_t s) {
     nelem_out.resize(n);
     row.resize(n + 1);
     elemrow.resize(n + 1);
-    queue.resize((size_t)n + 2);
+    queue.resize((size_t)n + kQueueIds);
     scan_ws.resize(scan_workspace_words(n));
     inited = true;
     computed = false;
@@ -644,11 +1170,10 @@ template <class S> void Ash3D<S>::compute(hipStream_t s) {
     if (!inited) throw std::invalid_argument("AlphaShape3D_compute called before init");
     Ash3Args<S> a = make_args3(*this);
     section_mark(s, kMarkCompute0);
-    fill<uint32_t>(queue.p, 2, 0u, s);
+    fill<uint32_t>(queue.p, kQueueIds, 0u, s);
     hipLaunchKernelGGL((fill3_kernel<S>), dim3(grid_for(n, 256)), dim3(256), 0, s, a);
     section_mark(s, kMarkFill);
-    hipLaunchKernelGGL((delaunay3_kernel<S>), dim3((n + kDelaunay3Block - 1) / kDelaunay3Block),
-                       dim3(kDelaunay3Block), 0, s, a);
+    launch_star3(a, s);
     section_mark(s, kMarkDelaunayMain);
     hipLaunchKernelGGL((delaunay3_exact_kernel<S>), dim3(kExactWaves3D), dim3(64), 0, s, a);
     section_mark(s, kMarkDelaunay);
@@ -668,7 +1193,9 @@ template <class S> void Ash3D<S>::compute(hipStream_t s) {
     computed = true;
 }
 
-template <class S> uint32_t Ash3D<S>::n_exact_nodes() { return computed ? read_scalar(queue.p) : 0u; }
+template <class S> uint32_t Ash3D<S>::n_exact_nodes() {
+    return computed ? read_scalar(queue.p) - read_scalar(queue.p + 2) : 0u;
+}
 template <class S> uint32_t Ash3D<S>::n_over_cap() { return computed ? read_scalar(queue.p + 1) : 0u; }
 
 template struct Ash3D<float>;

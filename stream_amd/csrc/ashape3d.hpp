@@ -14,14 +14,15 @@
 // ((t/64)*CAP + j)*64 + t%64: candidates (u32, CAP 124 = the reference's 128
 // minus the four infinity nodes), local tetrahedra (u32 packing three u8
 // local ids, CAP 256 >= 2*124 + 4 for a star of 124 link vertices) and
-// per-candidate counts (u8).  The cavity cycle lives in LDS, 128 bytes per
-// lane, as the reference's.
+// per-candidate counts (u8).  The insertion itself runs on registers and LDS,
+// 16 lanes per node; only the exact redo works in the slab.
 #pragma once
 #include "lbvh.hpp"
 
 namespace stream_amd {
 
 constexpr uint32_t kNInf3D = 4;
+constexpr uint32_t kQueueIds = 3;    // counters before the ids of the redo queue
 constexpr uint32_t kCand3D = 124;    // real candidates per node
 constexpr uint32_t kTet3D = 256;     // local tetrahedra per node
 constexpr uint32_t kCycle3D = 128;   // local ids (4 infinity + 124)
@@ -45,7 +46,7 @@ template <class S> struct Ash3D {
     DBuf<uint8_t> node_is_bnd, nelem, nelem_out;
     DBuf<uint32_t> neig, elemglob;
     DBuf<uint8_t> edge_is_bnd;
-    DBuf<uint32_t> queue;   // [0] = count, [1] = candidate overflows, then node ids
+    DBuf<uint32_t> queue;   // counts: redone, candidate overflows, redone for space; then node ids
     DBuf<uint64_t> scan_ws;
     uint32_t n_elems_ = 0, n_edges_ = 0;
     bool inited = false, computed = false;

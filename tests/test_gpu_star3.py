@@ -1,0 +1,67 @@
+"""The 16-lane local Delaunay of the 3D alpha-shape at the edges of its rules,
+bit for bit against the CPU oracle: node counts around a wavefront's four
+nodes, candidate lists from none to the clamped 124 (nodes that wait for room
+in the candidate pool), stars beyond 32 and beyond 64 tetrahedra, cavities
+beyond 14 and 32 and walks that the step cap stops, coordinates far from and
+close to 1 (FP32 tests that only the FP64 filter decides)."""
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+from stream_amd import clouds
+
+pytestmark = pytest.mark.gpu
+
+
+def _ball(n, seed):
+    """A centre and n points on the unit sphere, radii jittered by 1e-3: the
+    centre's star has about 2 n tetrahedra."""
+    rng = np.random.default_rng(seed)
+    v = rng.standard_normal((n, 3))
+    v *= ((1.0 + 1e-3 * rng.random(n)) / np.linalg.norm(v, axis=1))[:, None]
+    return np.concatenate([np.zeros((1, 3)), v])
+
+
+def _cloud(name):
+    kind, k = name.split("-")
+    k = int(k)
+    if kind == "random":  # few points, all candidates of each other
+        return np.random.default_rng(k).random((k, 3)), 2.0
+    if kind == "sparse":  # 0, 1, 2, ... candidates
+        return np.random.default_rng(k).random((k, 3)), 0.35 / k ** (1 / 3)
+    if kind == "ball":
+        return _ball(k, k), 3.0
+    if kind == "dense":  # alpha well above the spacing: clamped lists
+        return np.random.default_rng(k).random((k, 3)), 1.9 / k ** (1 / 3)
+    pts, al = clouds.sloshing_tank_scaled(k, 3)
+    return pts, 1.08 * al
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("name, scale, offset", [
+    ("random-4", 1.0, 0.0), ("random-5", 1.0, 0.0), ("random-7", 1.0, 0.0), ("random-33", 1.0, 0.0),
+    ("random-124", 1.0, 0.0), ("random-127", 1.0, 0.0), ("sparse-301", 1.0, 0.0), ("ball-17", 1.0, 0.0),
+    ("ball-34", 1.0, 0.0), ("ball-35", 1.0, 0.0), ("ball-60", 1.0, 0.0), ("ball-123", 1.0, 0.0),
+    ("dense-1500", 1.0, 0.0), ("dense-400", 2.0 ** -9, 0.0), ("dense-400", 2.0 ** 20, 0.0),
+    ("dense-400", 1.0, 300.0), ("tank-9000", 1.0, 0.0)])
+def test_outputs_match_oracle(name, scale, offset, dtype):
+    from stream_amd.mesh import AlphaShape3D
+
+    print(f"[star3] {name} x {scale} + {offset} {np.dtype(dtype).name}", flush=True)
+    pts, alpha = _cloud(name)
+    pts = ((pts + offset) * scale).astype(dtype)
+    al = np.broadcast_to(np.asarray(alpha * scale, dtype), len(pts)).copy()
+    o = ol.ashape3d(pts, al, bits=21, dtype=dtype)
+    a = AlphaShape3D(dtype=dtype, morton_bits=21)
+    a.set_nodes(pts, al)
+    a.compute()
+    row, neig, eb = a.get_edges()
+    assert np.array_equal(a.get_permutation(), o["perm"])
+    assert np.array_equal(row, o["row"])
+    assert np.array_equal(neig, o["neig"])
+    assert np.array_equal(eb, o["edge_is_bnd"])
+    assert np.array_equal(a.get_boundary_nodes(), o["node_is_bnd"])
+    assert np.array_equal(a.get_elem(), o["elem"])
+    if dtype == np.float64 and offset == 0.0:
+        # room alone never counts as an exact evaluation
+        assert a.get_nexact() <= o["n_exact_calls"]
