@@ -24,6 +24,10 @@ constexpr uint32_t kCounterWords = (1 + kMaxFoldGroups) * kCounterStride;
 // area, which the update kernel's fold must not overwrite while other
 // blocks of it still read them.
 constexpr size_t kJacobiDqSlot = 4ull * kMaxCgBlocks + 4ull * kMaxFoldGroups;
+// The one-kernel iteration's partials: the five sums of the even and the odd
+// states.
+constexpr size_t kCg1Slot = kJacobiDqSlot + kMaxCgBlocks;
+constexpr size_t kPartialsEnd = kCg1Slot + 10ull * kMaxCgBlocks;
 
 Tuning& tuning() {
     static Tuning t;
@@ -44,7 +48,8 @@ void CgWork::resize(uint32_t n, uint32_t nthreads) {
     if (blocks == 0) blocks = 1;
     sc.resize(1);
     out2.resize(2);
-    partials.resize(kJacobiDqSlot + kMaxCgBlocks);
+    partials.resize(kPartialsEnd);
+    hist.resize(2);
     if (!counter.p) {
         counter.resize(kCounterWords);
         fill<uint32_t>(counter.p, kCounterWords, 0u, ctx().stream);
@@ -65,14 +70,32 @@ void set_fold_group(uint32_t g) {
 
 namespace {
 
+// Sum over the wavefront, valid in lane 63: the prefix sums of a row of 16
+// lanes, then of the rows, on the data-parallel path of the ALU (a shuffle per
+// step goes through the LDS unit twice for a double and its latency is most of
+// a small kernel's reduction).
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum63(double v) {
+    v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+    v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+    v = dpp_add<0x118, 0xf>(v);  // row_shr:8
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // Block sum of an NT-thread block (s_tmp: NT / kWave doubles), valid in
 // thread 0.
 template <int NT> __device__ __forceinline__ double block_sum(double v, double* s_tmp) {
     constexpr uint32_t nw = NT / kWave;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    v = wave_sum63(v);
     const uint32_t w = threadIdx.x / kWave;
-    if (lane_id() == 0) s_tmp[w] = v;
+    if (lane_id() == kWave - 1) s_tmp[w] = v;
     __syncthreads();
     double t = 0.0;
     if (threadIdx.x == 0)
@@ -200,13 +223,9 @@ __device__ void store_partials(const double (&v)[K], double* __restrict__ p, uin
     __shared__ double s_w[K][nw];
     double a[K];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        a[k] = v[k];
-#pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) a[k] += __shfl_xor(a[k], o, kWave);
-    }
+    for (int k = 0; k < K; ++k) a[k] = wave_sum63(v[k]);
     const uint32_t wv = threadIdx.x / kWave;
-    if (lane_id() == 0)
+    if (lane_id() == kWave - 1)
 #pragma unroll
         for (int k = 0; k < K; ++k) s_w[k][wv] = a[k];
     __syncthreads();
@@ -227,8 +246,7 @@ __device__ __forceinline__ uint32_t flag_load(const uint32_t* p) {
 
 // The K x G partials a previous kernel stored with store_partials, read as
 // one index space e = k G + b: thread t adds entries t, t + NT, ...
-// of every k in ascending order, then the lanes' sums meet in an xor
-// butterfly (every lane gets the same bits, additions being commutative)
+// of every k in ascending order, then the lanes' sums meet in wave_sum63
 // and the waves' in LDS behind one barrier, in wave order.  Every block
 // that sums the same partials therefore gets the same bits, so each block
 // of a kernel can derive the same scalar (alpha, beta) without a grid-wide
@@ -249,11 +267,9 @@ template <int K, int NT> __device__ void finish_partials(double (&a)[K], double 
     constexpr uint32_t nw = NT / kWave;
     __shared__ double s_w[K][nw];
 #pragma unroll
-    for (int k = 0; k < K; ++k)
-#pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) a[k] += __shfl_xor(a[k], o, kWave);
+    for (int k = 0; k < K; ++k) a[k] = wave_sum63(a[k]);
     const uint32_t wv = threadIdx.x / kWave;
-    if (lane_id() == 0)
+    if (lane_id() == kWave - 1)
 #pragma unroll
         for (int k = 0; k < K; ++k) s_w[k][wv] = a[k];
     __syncthreads();
@@ -292,25 +308,25 @@ __device__ void sum_partials(const double* __restrict__ p, uint32_t stride, uint
 // point of use, two loads per round so that the caller's registers stay
 // few.  Both orders give sum_partials' bits.
 constexpr int kPrefetch = 4;
-struct PartialsPrefetch {
-    double v[kPrefetch];
+template <int P = kPrefetch> struct PartialsPrefetch {
+    double v[P];
     bool whole;
 };
-template <int K, int NT>
-__device__ __forceinline__ PartialsPrefetch prefetch_partials(const double* __restrict__ p, uint32_t stride,
+template <int K, int NT, int P = kPrefetch>
+__device__ __forceinline__ PartialsPrefetch<P> prefetch_partials(const double* __restrict__ p, uint32_t stride,
                                                               uint32_t G) {
-    PartialsPrefetch f;
+    PartialsPrefetch<P> f;
     const uint32_t total = K * G;
-    f.whole = total <= kPrefetch * NT;
+    f.whole = total <= P * NT;
 #pragma unroll
-    for (int u = 0; u < kPrefetch; ++u) {
+    for (int u = 0; u < P; ++u) {
         const uint32_t e = threadIdx.x + u * NT;
         f.v[u] = (f.whole && e < total) ? partial_at<K>(p, stride, G, e) : 0.0;
     }
     return f;
 }
-template <int K, int NT>
-__device__ void sum_prefetched(const PartialsPrefetch& f, const double* __restrict__ p, uint32_t stride, uint32_t G,
+template <int K, int NT, int P = kPrefetch>
+__device__ void sum_prefetched(const PartialsPrefetch<P>& f, const double* __restrict__ p, uint32_t stride, uint32_t G,
                                double (&tot)[K]) {
     if (!f.whole) {
         sum_partials<K, NT, 2>(p, stride, G, tot);
@@ -320,7 +336,7 @@ __device__ void sum_prefetched(const PartialsPrefetch& f, const double* __restri
 #pragma unroll
     for (int k = 0; k < K; ++k) a[k] = 0.0;
 #pragma unroll
-    for (int u = 0; u < kPrefetch; ++u) {
+    for (int u = 0; u < P; ++u) {
         const uint32_t e = threadIdx.x + u * NT;
         if (e < K * G) add_partial<K>(a, G, e, f.v[u]);
     }
@@ -871,6 +887,174 @@ __global__ __launch_bounds__(NT) void cg_update_kernel(uint32_t n, XV* __restric
     }
 }
 
+// One iteration in one kernel, for the Jacobi and the unpreconditioned solver:
+// predict-and-recompute CG (T. Chen and E. Carson, "Predict-and-Recompute
+// Conjugate Gradient Variants", SIAM J. Sci. Comput. 42, 2020).  With u =
+// M^-1 r and s = A p, every scalar comes from sums that one pass over the
+// vectors of a state gives, nu = u.r, mu = p.s, delta = u.s and gamma = s.M^-1 s:
+//   alpha = nu / mu, beta = (nu - 2 alpha delta + alpha^2 gamma) / nu
+// (the numerator is the next nu, expanded; alpha uses the recomputed one), then
+//   x += alpha p, u -= alpha M^-1 s, p = u + beta p, s = A p.
+// cg_dir / cg_update wait for the grid twice per iteration.  Here a row forms
+// its neighbours' new p itself from one record {u, M^-1 s, p} each (their
+// owners' operations, so the same bits), and the grid is waited for once,
+// between launches.  s is a product in every iteration, as in plain CG, so
+// the residual drifts no faster: iteration counts are the two-kernel ones' to
+// a few in a thousand (forms with a recursion for s failed on FP32 systems
+// that plain CG solves).  Bound: the launch and the chain entries -> records ->
+// sums, not bytes.  State k lives in record buffer, partials and history k & 1,
+// so that no kernel writes what another block of it still reads; every block
+// derives the same scalars and stop decision from the same partials.  x lags:
+// state k's x is complete once kernel k has run.
+template <class V> struct alignas(4 * sizeof(V)) CgRec {
+    V u, us, p, pad;
+};
+template <class V> struct CgRow {
+    V u, us, p;
+};
+template <class V> __device__ __forceinline__ CgRow<V> cg1_load(const CgRec<V>* rec, uint32_t i) {
+    return {rec[i].u, rec[i].us, rec[i].p};
+}
+
+// The sums of a state, a row's part; acc = (A p)_i, r = u / M^-1.
+template <class V, bool DIFF, int PREC>
+__device__ __forceinline__ void cg1_sums(double (&v)[5], V u, V us, V p, V acc, V diag, V idiag) {
+    const double r = PREC == kPrecNone ? (double)u : (DIFF ? (double)u / (double)idiag : (double)diag * (double)u);
+    v[0] += r * (double)u;
+    v[1] += (double)acc * (double)p;
+    v[2] += (double)acc * (double)u;
+    v[3] += (double)acc * (double)us;
+    v[4] += r * r;
+}
+
+constexpr int kCg1Prefetch = 8;  // 5 x G partials, G <= 409 blocks of 256 or 819 of 512
+template <class V, bool DIFF, int PREC, int CH, int NT>
+__global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restrict__ idiag,
+                                                 const CgRec<V>* __restrict__ cur, CgRec<V>* __restrict__ nxt,
+                                                 double* __restrict__ x, CgScalars* sc, Cg1Hist* hist,
+                                                 double* partials, uint32_t par) {
+    const uint32_t done = flag_load(&sc->done);
+    const Cg1Hist h = hist[par];
+    const double* pin = partials + kCg1Slot + (size_t)par * 5 * kMaxCgBlocks;
+    const auto pf = prefetch_partials<5, NT, kCg1Prefetch>(pin, kMaxCgBlocks, gridDim.x);
+    const uint32_t lane = threadIdx.x & 63u;
+    const SliceSpan sp = slice_span(M.nslices, M.map);
+    // the first slice's own records, entries and gathers before the sum
+    SliceRows<1> rows = slice_rows<V, 1>(M, sp.s, sp, lane);
+    uint32_t seg = rows.base[0];
+    CgRow<V> own = cg1_load(cur, rows.ii[0]);
+    V a[CH];
+    CgRow<V> g[CH];
+    auto load = [&](uint32_t k) {
+        uint32_t c[CH];
+        sell_load<V, CH>(M, seg, k, rows.L[0], rows.ii[0], c, a);
+#pragma unroll
+        for (int q = 0; q < CH; ++q) g[q] = cg1_load(cur, c[q]);
+    };
+    load(0);
+    if (done) return;
+    double tot[5];
+    sum_prefetched<5, NT, kCg1Prefetch>(pf, pin, kMaxCgBlocks, gridDim.x, tot);
+    const bool first_thread = blockIdx.x == 0 && threadIdx.x == 0;
+    // FP32 vectors: the recursion goes on to 0.6 of the tolerance (3% more
+    // iterations at 1e-8), so that the true residual, which its rounding moves
+    // by several percent, meets the tolerance at the first look
+    const double tol2 = sizeof(V) == 4 ? 0.36 * sc->tol2 : sc->tol2;
+    // (a state straight from the residual kernel was tested there)
+    if (!h.fresh && ((sc->crit ? tot[0] : tot[4]) <= tol2 || h.iter >= sc->maxit)) {
+        if (first_thread) {
+            sc->rr = tot[4];
+            sc->rz = tot[0];
+            sc->done = 1u;
+        }
+        return;
+    }
+    const double alpha = tot[0] / tot[1];
+    const double nu = tot[0] - 2.0 * alpha * tot[2] + alpha * alpha * tot[3];
+    const double beta = fmax(nu, 0.0) / tot[0];
+    if (first_thread) {
+        hist[par ^ 1u] = {h.iter + 1, 0u};
+        sc->rr = tot[4];
+        sc->rz = tot[0];
+        sc->alpha = alpha;
+        sc->beta = beta;
+        sc->iter = h.iter + 1;
+    }
+    const V av = (V)alpha, bv = (V)beta;
+    double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (uint32_t s0 = sp.s;;) {
+        const uint32_t i = rows.ii[0];
+        const V un = own.u - av * own.us, pn = un + bv * own.p, dg = M.diag[i];
+        V acc = dg * pn;
+        for (uint32_t k = 0;;) {
+#pragma unroll
+            for (int q = 0; q < CH; ++q) {
+                const V pj = (g[q].u - av * g[q].us) + bv * g[q].p;
+                acc = DIFF ? acc + a[q] * (pj - pn) : acc + a[q] * pj;
+            }
+            k += CH;
+            if (k >= rows.W) break;
+            load(k);
+        }
+        if (rows.valid[0]) {
+            const V id = PREC == kPrecJacobi ? idiag[i] : (V)1;
+            const V us = id * acc;
+            nxt[i].u = un;
+            nxt[i].us = us;
+            nxt[i].p = pn;
+            x[i] += alpha * (double)own.p;
+            cg1_sums<V, DIFF, PREC>(v, un, us, pn, acc, dg, id);
+        }
+        s0 += sp.step;
+        if (s0 >= sp.e) break;
+        rows = slice_rows<V, 1>(M, s0, sp, lane);
+        seg = rows.base[0];
+        own = cg1_load(cur, rows.ii[0]);
+        load(0);
+    }
+    store_partials<5, NT>(v, partials + kCg1Slot + (size_t)(par ^ 1u) * 5 * kMaxCgBlocks, kMaxCgBlocks);
+}
+
+// The state behind a residual kernel (r given): u = M^-1 r, and p = u at the
+// start; a replacement keeps the direction and beta, p += u - u_old.
+template <class V, int PREC, int NT>
+__global__ __launch_bounds__(NT) void cg1_start_kernel(uint32_t n, const V* __restrict__ idiag,
+                                                       const V* __restrict__ r, CgRec<V>* __restrict__ rec,
+                                                       Cg1Hist* hist, uint32_t par, bool replaced) {
+    CG_ROWS(i) {
+        const V un = PREC == kPrecJacobi ? idiag[i] * r[i] : r[i];
+        rec[i].p = replaced ? rec[i].p + (un - rec[i].u) : un;
+        rec[i].u = un;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (!replaced) hist[par].iter = 0u;
+        hist[par].fresh = 1u;
+    }
+}
+// s = A p of that state (in place: only p is read from other rows) and its
+// sums.
+template <class V, bool DIFF, int PREC, int CH, int NT>
+__global__ __launch_bounds__(NT) void cg1_apply_kernel(SellArgs<V> M, const V* __restrict__ idiag, CgRec<V>* rec,
+                                                       double* partials, uint32_t par) {
+    const uint32_t lane = threadIdx.x & 63u;
+    double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    SELL_FOR_SLICE_ROWS(1, rows) {
+        const uint32_t i = rows.ii[0];
+        const V pn = rec[i].p, dg = M.diag[i];
+        V acc[1] = {dg * pn};
+        sell_rows_product<V, 1, CH, V>(
+            M, rows, acc, [&](uint32_t j) -> V { return rec[j].p; },
+            [&](int, V ac, V a, V gj) { return DIFF ? ac + a * (gj - pn) : ac + a * gj; });
+        if (rows.valid[0]) {
+            const V id = PREC == kPrecJacobi ? idiag[i] : (V)1;
+            const V us = id * acc[0];
+            rec[i].us = us;
+            cg1_sums<V, DIFF, PREC>(v, rec[i].u, us, pn, acc[0], dg, id);
+        }
+    }
+    store_partials<5, NT>(v, partials + kCg1Slot + (size_t)par * 5 * kMaxCgBlocks, kMaxCgBlocks);
+}
+
 // L L^T path, one kernel for the update and the first half of the apply:
 // x += alpha d; r' = r - alpha q; w = L^T r' (w_i = L_ii r'_i + sum_{j>i}
 // L_ji r'_j, U = the upper SELL).  r and q live interleaved ({r, q} per
@@ -895,7 +1079,7 @@ __global__ __launch_bounds__(NT) void llt_update_kernel(SellArgs<V> U, XV* __res
     const bool it = mode == 0;
     // the direction kernel's partials and the first slice group's own data
     // are loaded before the partials' sum (alpha) is taken
-    PartialsPrefetch pf{};
+    PartialsPrefetch<> pf{};
     if (it) pf = prefetch_partials<1, NT>(partials, kMaxCgBlocks, gridDim.x);
     const uint32_t lane = threadIdx.x & 63u;
     const SliceSpan sp = slice_span(M.nslices, M.map);
@@ -980,7 +1164,7 @@ __global__ __launch_bounds__(NT) void llt_lo_kernel(SellArgs<V> M, const V* __re
     const uint32_t done = mode == 0 ? flag_load(&sc->done) : 0u;
     // the partials' loads go out first; their sum (beta) is taken after the
     // wavefront's first slice group, whose loads cover their latency
-    const PartialsPrefetch pf = prefetch_partials<2, NT>(partials + kMaxCgBlocks, kMaxCgBlocks, gridDim.x);
+    const PartialsPrefetch<> pf = prefetch_partials<2, NT>(partials + kMaxCgBlocks, kMaxCgBlocks, gridDim.x);
     const uint32_t lane = threadIdx.x & 63u;
     const SliceSpan sp = slice_span(M.nslices, M.map);
     auto product = [&](const SliceRows<R>& rows, V (&acc)[R]) {
@@ -1122,7 +1306,7 @@ template <class V> CgVecs<V> carve(CgWork& w, uint32_t n) {
 // is rough on the mesh scale, which A amplifies against the smooth
 // right-hand side (16% more iterations on the 1M dam-break).
 // ---------------------------------------------------------------------------
-template <class V, bool DIFF, int PREC, int CH, int R, int NT>
+template <class V, bool DIFF, int PREC, int CH, int R, int NT, bool ONE = false>
 void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const LowerFactor<V>* L, const double* b,
               double* x, const CgOptions& o, CgWork& w, SolveStats& st, hipStream_t s) {
     using XV = double;
@@ -1162,8 +1346,17 @@ void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const
             hipLaunchKernelGGL((cg_residual_kernel<V, PREC, NT, 8>), grid, blk, 0, s, n, A64.row.p, A64.col.p,
                                A64.val.p, b, x, rp, rs, cur, idiag, w.sc.p, w.partials.p, w.counter.p, mode, rtol2);
     };
+    CgRec<V>* rec[2] = {reinterpret_cast<CgRec<V>*>(vv.P[0]), reinterpret_cast<CgRec<V>*>(vv.RQ[0])};
     auto residual = [&](int mode, uint32_t it) {
         V2<V>* cur = vv.P[it & 1];
+        if constexpr (ONE) {
+            residual_kernel(vv.r, 1u, reinterpret_cast<V2<V>*>(vv.D[0]), mode);
+            hipLaunchKernelGGL((cg1_start_kernel<V, PREC, NT>), grid, blk, 0, s, n, idiag, vv.r, rec[it & 1],
+                               w.hist.p, it & 1u, mode != 0);
+            hipLaunchKernelGGL((cg1_apply_kernel<V, DIFF, PREC, CH, NT>), grid, blk, 0, s, MA, idiag, rec[it & 1],
+                               w.partials.p, it & 1u);
+            return;
+        }
         if constexpr (PREC == kPrecLLt) {
             V2<V>* rqc = vv.RQ[it & 1];
             residual_kernel(reinterpret_cast<V*>(rqc), 2u, cur, mode);
@@ -1180,6 +1373,11 @@ void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const
     auto launch_batch = [&](uint32_t it0) {
         for (uint32_t k = 0; k < o.batch; ++k) {
             const uint32_t it = it0 + k;
+            if constexpr (ONE) {
+                hipLaunchKernelGGL((cg1_kernel<V, DIFF, PREC, CH, NT>), grid, blk, 0, s, MA, idiag, rec[it & 1],
+                                   rec[(it + 1) & 1], xacc, w.sc.p, w.hist.p, w.partials.p, it & 1u);
+                continue;
+            }
             V2<V>* cur = vv.P[it & 1];
             V2<V>* nxt = vv.P[(it + 1) & 1];
             if constexpr (PREC == kPrecLLt) {
@@ -1298,25 +1496,57 @@ void cg_solve_llt(const DevCsr<double>& A64, const Sell<V>& S, const LowerFactor
         cg_drive<V, DIFF, kPrecLLt, CH, 1, 1024>(A64, S, nullptr, L, b, x, o, w, st, s);
 }
 
+// Block size of the one-kernel iteration of values V on n rows (0: the
+// two-kernel one).  us per iteration, two kernels -> one, FP64: 2D 11.9 -> 7.6
+// (16k rows), 12.1 -> 8.3 (60k), 13.7 -> 9.9 (90k), 14.1 -> 10.7 (130k), 14.9
+// -> 17.5 (150k); 3D 15.0 -> 12.0 (30k), 18.1 -> 17.1 (120k), 23.8 -> 30.2
+// (200k).  FP32: 2D 12.3 -> 7.9 (60k), 13.9 -> 11.7 (150k), 3D 17.6 -> 14.1
+// (120k), 19.8 -> 18.3 (200k), 23.8 -> 28.1 (300k).  The line is where CUs get a
+// second block (FP64: 32-byte records, 12 wavefronts per CU) or where the
+// records' gathers cost more than the second launch.  One block per CU as
+// far as 256 threads allow that: 7.2 against 8.2 us with 512 at 16k.
+template <class V> uint32_t cg1_threads(uint32_t n) {
+    if (n > (sizeof(V) == 8 ? 256u : 384u) * 512u) return 0;
+    return n <= 256u * 256u ? 256 : 512;
+}
+
 template <class V, int CH>
 void cg_solve_ch(const DevCsr<double>& A64, const Sell<V>& S, bool diff, int32_t prec, const V* idiag,
                  const LowerFactor<V>* L, const double* b, double* x, const CgOptions& o, CgWork& w,
                  SolveStats& st, hipStream_t s) {
     constexpr int NT = kCgThreads;
-    if (diff) {
-        if (prec == kPrecLLt)
+    if (prec == kPrecLLt) {
+        if (diff)
             cg_solve_llt<V, true, CH>(A64, S, L, b, x, o, w, st, s);
-        else if (prec == kPrecJacobi)
-            cg_drive<V, true, kPrecJacobi, CH, 1, NT>(A64, S, idiag, L, b, x, o, w, st, s);
         else
-            cg_drive<V, true, kPrecNone, CH, 1, NT>(A64, S, idiag, L, b, x, o, w, st, s);
-    } else {
-        if (prec == kPrecLLt)
             cg_solve_llt<V, false, CH>(A64, S, L, b, x, o, w, st, s);
-        else if (prec == kPrecJacobi)
-            cg_drive<V, false, kPrecJacobi, CH, 1, NT>(A64, S, idiag, L, b, x, o, w, st, s);
+        return;
+    }
+    auto go = [&](auto d, auto p) {
+        constexpr bool D = decltype(d)::value;
+        constexpr int P = decltype(p)::value;
+        // (without the true residual's verdict the result is the recursion's
+        // own: those callers keep the two-kernel one)
+        const uint32_t one = o.verify ? cg1_threads<V>(A64.n) : 0u;
+        if (one == 256)
+            cg_drive<V, D, P, CH, 1, 256, true>(A64, S, idiag, L, b, x, o, w, st, s);
+        else if (one == 512)
+            cg_drive<V, D, P, CH, 1, 512, true>(A64, S, idiag, L, b, x, o, w, st, s);
         else
-            cg_drive<V, false, kPrecNone, CH, 1, NT>(A64, S, idiag, L, b, x, o, w, st, s);
+            cg_drive<V, D, P, CH, 1, NT>(A64, S, idiag, L, b, x, o, w, st, s);
+    };
+    using Jac = std::integral_constant<int, kPrecJacobi>;
+    using Non = std::integral_constant<int, kPrecNone>;
+    if (diff) {
+        if (prec == kPrecJacobi)
+            go(std::true_type{}, Jac{});
+        else
+            go(std::true_type{}, Non{});
+    } else {
+        if (prec == kPrecJacobi)
+            go(std::false_type{}, Jac{});
+        else
+            go(std::false_type{}, Non{});
     }
 }
 

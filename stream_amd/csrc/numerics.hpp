@@ -96,9 +96,16 @@ struct CgScalars {
     uint32_t pad[2];
 };
 
+// State k of the one-kernel iteration.
+struct Cg1Hist {
+    uint32_t iter;   // k
+    uint32_t fresh;  // the residual kernel tested this state already
+};
+
 struct CgWork {
     DBuf<CgScalars> sc;
-    DBuf<double> partials;   // [3][blocks]
+    DBuf<Cg1Hist> hist;
+    DBuf<double> partials;   // block partials, by kernel
     DBuf<uint32_t> counter;  // last-block tickets
     DBuf<double> out2;       // true-residual norms
     DBuf<uint8_t> vbuf;      // solver vectors (grow-only)

@@ -1,0 +1,122 @@
+"""The one-kernel Jacobi-PCG iteration at the edges of its rule: row counts
+around a wavefront, a block, the 256 / 512 thread blocks and the two-kernel
+iteration, rows from empty to wider than one load step, a starting guess, the
+iteration cap, and graph replay.  Oracle: textbook FP64 PCG and the FP64
+residual b - A x, both in numpy / scipy."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _band(n, width, seed=0):
+    """SPD, diagonally dominant, rows of 0 to 2 width off-diagonals."""
+    rng = np.random.default_rng(seed + n)
+    offs = [k for k in range(1, width + 1) if k < n]
+    parts = []
+    for k in offs:
+        w = rng.random(n - k) * (rng.random(n - k) < 0.7)
+        parts.append(sp.diags(-w, k, shape=(n, n)))
+    U = sum(parts[1:], parts[0]) if parts else sp.csr_matrix((n, n))
+    A = (U + U.T).tocsr()
+    A.eliminate_zeros()
+    A = (A + sp.diags(0.02 + rng.random(n) * 0.05 - np.asarray(A.sum(1)).ravel())).tocsr()
+    A.sort_indices()
+    return A
+
+
+def _system(A, b):
+    from stream_amd.numerics import DeviceCSR, HostCSR, LinSys, PrecJacobi
+
+    d = DeviceCSR(HostCSR(A.indptr.astype(np.uint32), A.indices.astype(np.uint32), A.data.astype(np.float64)))
+    return LinSys(d, b), PrecJacobi(d)
+
+
+def _rel(A, b, x):
+    return np.linalg.norm(b - A @ x) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("n, width", [(1, 1), (2, 1), (63, 3), (64, 3), (65, 4), (256, 9), (257, 4), (1000, 20),
+                                      (65_536, 3), (65_537, 3), (131_072, 3), (131_073, 3), (196_608, 2),
+                                      (196_609, 2)])
+def test_solves_to_the_true_residual(n, width, mixed):
+    from stream_amd.numerics import SolverCG
+
+    print(f"[cg one] n={n} width={width} mixed={mixed}", flush=True)
+    A = _band(n, width)
+    rng = np.random.default_rng(3)
+    b = rng.standard_normal(n)
+    s, prec = _system(A, b)
+    x = rng.standard_normal(n)  # a starting guess
+    it, rel = (SolverCG().solve_mixed if mixed else SolverCG().solve_rel)(s, prec, x, rtol=1e-9)
+    assert _rel(A, b, x) <= 1e-9 * (1 + 1e-6) and abs(rel - _rel(A, b, x)) <= 1e-12
+    if not mixed:
+        # the same iterates in exact arithmetic
+        x0 = np.zeros(n)
+        it0, _ = SolverCG().solve_rel(s, prec, x0, rtol=1e-9)
+        _, ito, _ = O.jacobi_pcg(A.indptr.astype(np.uint32), A.indices.astype(np.uint32), A.data, b, rtol=1e-9)
+        assert abs(it0 - ito) <= 2
+
+
+def test_iteration_cap_is_exact():
+    from stream_amd import StreamError
+    from stream_amd.numerics import SolverCG
+
+    A = _band(5000, 1)
+    b = np.ones(5000)
+    s, prec = _system(A, b)
+    errs = []
+    for cap in (1, 31, 32, 33, 64):
+        x = np.zeros(5000)
+        with pytest.raises(StreamError):
+            SolverCG().solve_rel(s, prec, x, rtol=1e-15, maxit=cap)
+        # plain CG's iterate after `cap` steps
+        y, r = np.zeros(5000), b.copy()
+        dg = A.diagonal()
+        z = r / dg
+        d, rz = z.copy(), r @ z
+        for _ in range(cap):
+            q = A @ d
+            al = rz / (d @ q)
+            y += al * d
+            r = r - al * q
+            z = r / dg
+            rz, be = r @ z, (r @ z) / rz
+            d = z + be * d
+        errs.append(np.linalg.norm(x - y) / np.linalg.norm(y))
+    print("[cg one] cap errors", errs, flush=True)
+    assert max(errs) < 1e-10
+
+
+def test_zero_right_hand_side():
+    from stream_amd.numerics import SolverCG
+
+    A = _band(300, 2)
+    s, prec = _system(A, np.zeros(300))
+    x = np.zeros(300)
+    SolverCG().solve_rel(s, prec, x, rtol=1e-8)
+    assert np.array_equal(x, np.zeros(300))
+
+
+def test_graph_replay_gives_the_same_bits():
+    from stream_amd import tune
+    from stream_amd.numerics import SolverCG
+
+    A = _band(20_000, 3)
+    b = np.random.default_rng(5).standard_normal(20_000)
+    s, prec = _system(A, b)
+    xs = []
+    for graph in (0, 1, 1, 0):
+        tune("graph", graph)
+        try:
+            x = np.zeros(20_000)
+            SolverCG().solve_mixed(s, prec, x, rtol=1e-9)
+        finally:
+            tune("graph", 0)
+        xs.append(x)
+    for x in xs[1:]:
+        assert np.array_equal(x, xs[0])
