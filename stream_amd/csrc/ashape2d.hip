@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "ashape2d.hpp"
+#include "candidates.hpp"
 #include "predicates.hpp"
 
 namespace stream_amd {
@@ -143,6 +144,47 @@ template <class S> __global__ __launch_bounds__(256) void fill_kernel(AshArgs<S>
         if (nloc > kMaxFill2D) break;
     }
     a.nineig[tid] = nloc;
+}
+// The same by 8 lanes per node (candidates.hpp).  A node with more than
+// kMaxFill2D entries keeps those of the visits up to that point (cpp:351).
+constexpr int kFillLanes2D = 8, kFillStack2D = 96;
+constexpr uint32_t kFillBlock = 256, kMostCand2D = kMaxFill2D - kNInf2D;
+template <class S> __global__ __launch_bounds__(kFillBlock) void fill_group_kernel(AshArgs<S> a, uint32_t blocks_per_xcd) {
+    constexpr uint32_t G = kFillLanes2D, NPB = kFillBlock / G;
+    __shared__ CandStack<kFillStack2D> lds[NPB];
+    const uint32_t sub = threadIdx.x % G, slot = threadIdx.x / G, grp = slot % (64 / G);
+    const uint32_t tid = ((blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3)) * NPB + slot;
+    if (tid >= a.n) return;
+    const CandTree<S, 2> t{a.n, a.P, a.node, a.ibox};
+    const Sph4<S> si = a.P[tid];
+    const S two_delta = Consts2D<S>::two_delta;
+    auto store = [&](uint32_t j, uint32_t c) {
+        if (j < kMostCand2D + 2) a.cand[slab_index(tid, j)] = c;
+    };
+    uint32_t found = 0;
+    const bool done = cand_group<S, 2, (int)G>(t, tid, si, two_delta, sub, grp, lds[slot], kMostCand2D, &found, store);
+    if ((!done || found > kMostCand2D) && sub == 0) {
+        found = 0;
+        cand_walk(t, tid, si, two_delta, a.flags, [&](uint32_t c) {
+            store(found++, c);
+            return found <= kMostCand2D;
+        });
+    }
+    if (sub == 0) a.nineig[tid] = kNInf2D + found;
+}
+// Up to here one lane per node leaves the chip waiting for its walks (us, one
+// lane -> 8, FP32 dam-break: 81 -> 28 at 4k nodes, 92 -> 52 at 65k, 111 -> 106
+// at 160k); beyond, what the 8 lanes do for nothing costs more (157 -> 180 at
+// 300k, 489 -> 586 at 1M).
+constexpr uint32_t kFillGroupMax = 196608;
+template <class S> void launch_fill(const AshArgs<S>& a, hipStream_t s) {
+    if (a.n > kFillGroupMax) {
+        hipLaunchKernelGGL((fill_kernel<S>), dim3((a.n + kFillBlock - 1) / kFillBlock), dim3(kFillBlock), 0, s, a);
+        return;
+    }
+    constexpr uint32_t nodes = kFillBlock / kFillLanes2D;
+    const uint32_t per_xcd = ((a.n + nodes - 1) / nodes + 7) / 8;
+    hipLaunchKernelGGL((fill_group_kernel<S>), dim3(8 * per_xcd), dim3(kFillBlock), 0, s, a, per_xcd);
 }
 
 __device__ __forceinline__ uint16_t pack_tri(uint32_t a, uint32_t b) { return (uint16_t)(a | (b << 8)); }
@@ -596,7 +638,7 @@ template <class S> void Ash2D<S>::compute(hipStream_t s) {
     AshArgs<S> a = make_args(*this);
     section_mark(s, kMarkCompute0);
     fill<uint32_t>(queue.p, 1, 0u, s);
-    hipLaunchKernelGGL((fill_kernel<S>), dim3(grid_for(n, 256)), dim3(256), 0, s, a);
+    launch_fill(a, s);
     section_mark(s, kMarkFill);
     hipLaunchKernelGGL((delaunay_kernel<S>), dim3(grid_for(n, 256)), dim3(256), 0, s, a);
     section_mark(s, kMarkDelaunayMain);

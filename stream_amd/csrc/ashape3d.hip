@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "ashape3d.hpp"
+#include "candidates.hpp"
 #include "predicates.hpp"
 
 namespace stream_amd {
@@ -61,94 +62,34 @@ template <class S> __global__ void infinity3_kernel(const BoxD<S, 3>* gbox, Sph4
     P[n + 3] = p;
 }
 
-// Candidate search (cpp:310-363): stack DFS, children in order, leaves
-// tested when their parent is visited; the first 124 candidates are kept
-// (the reference clamps its list to 128 entries including the 4 infinity
-// nodes and warns), queue[1] counts clamped nodes.
-//
-// The DFS pushes the hit children of a node in order and pops the last one
-// pushed.  Here that last child is kept in a register instead of going
-// through the stack, and an internal child's node word is loaded with its
-// box, so descending costs one round of loads; the stack (63 entries + the
-// register = the 64-deep stack; the first 16 levels in LDS, laid out level
-// by level so that the lanes' words are consecutive, the rest in private
-// memory) holds node words, so a pop needs no node load.  The visit order, and so the candidate order, is
-// that of the plain push/pop loop, and so is the capacity error.
-constexpr int kFillLds = 16;  // stack levels held in LDS ([level][thread]); deeper ones in private memory
-template <class S> __global__ __launch_bounds__(256) void fill3_kernel(Ash3Args<S> a) {
-    __shared__ uint32_t lstack[kFillLds][256];
-    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
+// Candidate search (candidates.hpp), 16 lanes per node.  The first 124
+// candidates are kept (the reference clamps its list to 128 entries including
+// the 4 infinity nodes and warns), queue[1] counts clamped nodes.
+constexpr int kFillLanes3D = 16, kFillStack3D = 192;
+constexpr uint32_t kFillBlock = 256;
+template <class S> __global__ __launch_bounds__(kFillBlock) void fill3_kernel(Ash3Args<S> a, uint32_t blocks_per_xcd) {
+    constexpr uint32_t G = kFillLanes3D, NPB = kFillBlock / G;
+    __shared__ CandStack<kFillStack3D> lds[NPB];
+    const uint32_t sub = threadIdx.x % G, slot = threadIdx.x / G, grp = slot % (64 / G);
+    const uint32_t tid = ((blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3)) * NPB + slot;
     if (tid >= a.n) return;
+    const CandTree<S, 3> t{a.n, a.P, a.node, a.ibox};
     const Sph4<S> si = a.P[tid];
     const S two_delta = Consts3D<S>::two_delta;
-    const S rs = two_delta * si.r;
-    uint32_t stack[63 - kFillLds];
-    int ss = 0;
-    bool live = a.n >= 2;
-    uint32_t w = live ? a.node[0] : 0u;
-    uint32_t nloc = 0;
-    bool over = false;
-    for (uint32_t visits = 0; live && !over; ++visits) {
-        if (visits >= a.n) {
-            raise_flag(a.flags, kErrCapacity);
-            break;
-        }
-        const uint32_t sep = w & 0x3fffffffu;
-        const uint32_t cl = w >> 30;
-        bool hit[2] = {false, false};
-        uint32_t wc[2] = {0u, 0u};
-#pragma unroll
-        for (uint32_t ch = 0; ch < 2; ++ch) {
-            const uint32_t c = sep + ch;
-            if (!(cl & (ch + 1))) {
-                const BoxD<S, 3> bb = a.ibox[c];
-                wc[ch] = a.node[c];
-                const S dmaxx = fmax(si.c[0] - bb.hi[0], (S)0);
-                const S dmaxy = fmax(si.c[1] - bb.hi[1], (S)0);
-                const S dmaxz = fmax(si.c[2] - bb.hi[2], (S)0);
-                const S dminx = fmax(bb.lo[0] - si.c[0], (S)0);
-                const S dminy = fmax(bb.lo[1] - si.c[1], (S)0);
-                const S dminz = fmax(bb.lo[2] - si.c[2], (S)0);
-                hit[ch] =
-                    dmaxx * dmaxx + dminx * dminx + dmaxy * dmaxy + dminy * dminy + dmaxz * dmaxz + dminz * dminz <
-                    rs * rs;
-            } else if (tid != c && !over) {
-                const Sph4<S> sj = a.P[c];
-                const S ma = fmin(si.r, sj.r);
-                const S dx = si.c[0] - sj.c[0], dy = si.c[1] - sj.c[1], dz = si.c[2] - sj.c[2];
-                const S sq = dx * dx + dy * dy + dz * dz;
-                if (sq < (two_delta * ma) * (two_delta * ma)) {
-                    if (nloc < kCand3D)
-                        a.cand[slab3(tid, nloc++, kCand3D)] = c;
-                    else
-                        over = true;
-                }
-            }
-        }
-        if (hit[0] && hit[1]) {
-            if (ss < 63) {
-                if (ss < kFillLds)
-                    lstack[ss][threadIdx.x] = wc[0];
-                else
-                    stack[ss - kFillLds] = wc[0];
-                ++ss;
-                w = wc[1];
-            } else {
-                // a full stack drops the second child and visits the first
-                raise_flag(a.flags, kErrCapacity);
-                w = wc[0];
-            }
-        } else if (hit[0] || hit[1]) {
-            w = hit[1] ? wc[1] : wc[0];
-        } else if (ss != 0) {
-            --ss;
-            w = ss < kFillLds ? lstack[ss][threadIdx.x] : stack[ss - kFillLds];
-        } else {
-            live = false;
-        }
+    auto store = [&](uint32_t j, uint32_t c) {
+        if (j < kCand3D) a.cand[slab3(tid, j, kCand3D)] = c;
+    };
+    uint32_t found = 0;
+    if (!cand_group<S, 3, (int)G>(t, tid, si, two_delta, sub, grp, lds[slot], kCand3D, &found, store) && sub == 0) {
+        found = 0;
+        cand_walk(t, tid, si, two_delta, a.flags, [&](uint32_t c) {
+            store(found++, c);
+            return found <= kCand3D;
+        });
     }
-    if (over) atomicAdd(&a.queue[1], 1u);
-    a.nineig[tid] = kNInf3D + nloc;
+    if (sub != 0) return;
+    if (found > kCand3D) atomicAdd(&a.queue[1], 1u);
+    a.nineig[tid] = kNInf3D + min(found, kCand3D);
 }
 
 template <class S> __device__ __forceinline__ void load3(const Sph4<S>* P, uint32_t i, S* p) {
@@ -158,6 +99,12 @@ template <class S> __device__ __forceinline__ void load3(const Sph4<S>* P, uint3
     p[2] = s.c[2];
 }
 
+// LDS written by other lanes of this wavefront: program order is execution
+// order there, so only the compiler has to be held.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 // Boundary of the R removed tetrahedra at positions Tlast .. Tlast + R - 1 of
 // T (cpp:497-580): Ray et al.'s cycle walk, C(v) = next vertex of v on the
 // cycle (kEmpty off it).  C must be kEmpty for every vertex of the star.
@@ -214,6 +161,71 @@ __device__ __forceinline__ bool cavity_walk(TF&& T, CF&& C, uint32_t Tlast, uint
     }
     *first_out = first;
     return Rsize != 0;
+}
+
+// Minimum over the wavefront.
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xf, 0xf, false));  // row_shr:2
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xf, 0xf, false));  // row_shr:4
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xf, 0xf, false));  // row_shr:8
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// cavity_walk by a whole wavefront, one removed triangle per lane (R <= 64):
+// every remaining triangle is tried at once, and the one at the lowest
+// position joins, as the scan would find it after one failed step per position
+// before.  T keeps its order (only the new tetrahedra follow).
+template <class TF, class CF>
+__device__ __forceinline__ bool wave_walk(TF&& T, CF&& C, uint32_t m, uint32_t R, uint32_t* first_out) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t tw = lane < R ? T(m + lane) : 0u, tl = T(m + R - 1);
+    const uint32_t x = tw & 255u, y = (tw >> 8) & 255u, z = (tw >> 16) & 255u;
+    const uint32_t ta = tl & 255u, tb = (tl >> 8) & 255u, tc = (tl >> 16) & 255u;
+    C(ta) = tb;
+    C(tb) = tc;
+    C(tc) = ta;
+    wave_lds_sync();
+    uint32_t first = ta, left = R - 1, steps = 0;
+    uint32_t pos = lane < R - 1 ? lane : ~0u;  // position behind m; ~0: in the cycle already
+    while (left) {
+        const uint32_t cx = C(x), cy = C(y), cz = C(z);
+        const bool o0 = cy == x, o1 = cz == y, o2 = cx == z;
+        const bool simple = (o0 || o1 || o2) && (o0 || o1 || cy == kEmpty) && (o1 || o2 || cz == kEmpty) &&
+                            (o2 || o0 || cx == kEmpty);
+        const uint32_t best = wave_min(simple ? pos : ~0u);
+        steps += best + 1;
+        if (best == ~0u || steps > 100) break;
+        const bool mine = pos == best;
+        uint32_t nf = first;  // another start when the first corner goes inside
+        wave_lds_sync();
+        if (mine) {
+            if (!o0) C(x) = y;
+            if (!o1) C(y) = z;
+            if (!o2) C(z) = x;
+            if (o0 && o1) {
+                nf = nf == y ? cy : nf;
+                C(y) = kEmpty;
+            }
+            if (o1 && o2) {
+                nf = nf == z ? cz : nf;
+                C(z) = kEmpty;
+            }
+            if (o2 && o0) {
+                nf = nf == x ? cx : nf;
+                C(x) = kEmpty;
+            }
+        }
+        const uint64_t chg = __builtin_amdgcn_ballot_w64(nf != first);
+        if (chg) first = (uint32_t)__builtin_amdgcn_readlane((int)nf, __builtin_ctzll(chg));
+        --left;
+        pos = mine ? ~0u : (pos == left ? best : pos);
+        wave_lds_sync();
+    }
+    *first_out = first;
+    return left != 0;
 }
 
 // The alpha filter of the tetrahedron (tid, i2, i3, i4) (cpp:590-682): kept
@@ -273,153 +285,226 @@ template <class S> __device__ __forceinline__ void empty_star(const Ash3Args<S>&
     a.nfneig[tid] = 0;
 }
 
-// Local Delaunay of node tid's star + alpha filter (cpp:380-682), one lane,
-// every undecided sign through the exact stage.
-template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, uint32_t tid, uint8_t* cyc, double* ws) {
-    const uint32_t n = a.n;
+// Local Delaunay of node tid's star + alpha filter (cpp:380-682) by one
+// wavefront, every undecided sign through the exact stage.  A lane tests the
+// tetrahedra at its positions (each is tested once per insertion, and its
+// result depends on it and the point alone, so the order is free); lane 0
+// evaluates the undecided ones, with the expansion in LDS.  Removal and
+// re-triangulation run on the flags, on every lane alike.
+template <class S> struct Exact3Lds {
+    double ws[kExactWs3D];
+    S x[kCycle3D][3];  // candidates
+    uint32_t t[kTet3D];
+    uint32_t c[kCycle3D];
+};
+template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, uint32_t tid, Exact3Lds<S>& L) {
+    const uint32_t n = a.n, lane = threadIdx.x & 63u;
     const Sph4<S>* P = a.P;
     const uint32_t ncand = a.nineig[tid];
     auto neig = [&](uint32_t j) -> uint32_t { return j < kNInf3D ? n + j : a.cand[slab3(tid, j - kNInf3D, kCand3D)]; };
-    auto T = [&](uint32_t ti) -> uint32_t& { return a.tet[slab3(tid, ti, kTet3D)]; };
-    auto C = [&](uint32_t v) -> uint8_t& { return cyc[v]; };
+    auto T = [&](uint32_t ti) -> uint32_t& { return L.t[ti]; };
+    auto C = [&](uint32_t v) -> uint32_t& { return L.c[v]; };
 
     T(0) = pack_tet(0, 2, 1);
     T(1) = pack_tet(1, 2, 3);
     T(2) = pack_tet(0, 1, 3);
     T(3) = pack_tet(0, 3, 2);
+    for (uint32_t j = lane; j < ncand; j += 64) load3(P, neig(j), L.x[j]);
+    wave_lds_sync();
     S pa0[3];
     load3(P, tid, pa0);
+    auto corner = [&](uint32_t j, S* p) {
+        p[0] = L.x[j][0];
+        p[1] = L.x[j][1];
+        p[2] = L.x[j][2];
+    };
     uint32_t Tlast = 4;
     bool over = false;
     for (uint32_t pi = kNInf3D; pi < ncand; ++pi) {
-        const uint32_t curr = neig(pi);
         S pe0[3];
-        load3(P, curr, pe0);
-        uint32_t Rsize = 0;
-        uint32_t ti = 0;
-        while (ti < Tlast) {
-            const uint32_t tl = T(ti);
-            const uint32_t la = tl & 255u, lb = (tl >> 8) & 255u, lc = (tl >> 16) & 255u;
-            uint32_t i2 = neig(la), i3 = neig(lb), i4 = neig(lc);
+        corner(pi, pe0);
+        uint64_t f[4] = {0, 0, 0, 0};
+#pragma unroll 1
+        for (uint32_t q = 0; q * 64 < Tlast; ++q) {
+            const uint32_t ti = q * 64 + lane;
             S pb[3], pc[3], pd[3];
-            load3(P, i2, pb);
-            load3(P, i3, pc);
-            load3(P, i4, pd);
-            S err;
-            S det = -insphere_filter(pa0, pb, pc, pd, pe0, &err);
-            if (!((det > err) || (-det > err))) {
-                uint32_t i1 = tid, i5 = curr;
-                S qa[3] = {pa0[0], pa0[1], pa0[2]}, qe[3] = {pe0[0], pe0[1], pe0[2]};
-                S* p1 = qa;
-                S* p2 = pb;
-                S* p3 = pc;
-                S* p4 = pd;
-                S* p5 = qe;
-                bool swap = false;
-                auto cs = [&](uint32_t& x, uint32_t& y, S*& px, S*& py) {
-                    if (x > y) {
-                        const uint32_t t = x;
-                        x = y;
-                        y = t;
-                        S* u = px;
-                        px = py;
-                        py = u;
-                        swap = !swap;
+            uint32_t tl = 0;
+            S det = (S)0;
+            bool undecided = false;
+            if (ti < Tlast) {
+                tl = T(ti);
+                corner(tl & 255u, pb);
+                corner((tl >> 8) & 255u, pc);
+                corner((tl >> 16) & 255u, pd);
+                S err;
+                det = -insphere_filter(pa0, pb, pc, pd, pe0, &err);
+                undecided = !((det > err) || (-det > err));
+            }
+            // one undecided lane after the other: the workspace is shared
+            uint64_t u = __builtin_amdgcn_ballot_w64(undecided);
+            for (; u; u &= u - 1) {
+                if (lane == (uint32_t)__builtin_ctzll(u)) {
+                    double* ws = L.ws;
+                    uint32_t i1 = tid, i2 = neig(tl & 255u), i3 = neig((tl >> 8) & 255u),
+                             i4 = neig((tl >> 16) & 255u), i5 = neig(pi);
+                    S qa[3] = {pa0[0], pa0[1], pa0[2]}, qe[3] = {pe0[0], pe0[1], pe0[2]};
+                    S* p1 = qa;
+                    S* p2 = pb;
+                    S* p3 = pc;
+                    S* p4 = pd;
+                    S* p5 = qe;
+                    bool swap = false;
+                    auto cs = [&](uint32_t& x, uint32_t& y, S*& px, S*& py) {
+                        if (x > y) {
+                            const uint32_t t = x;
+                            x = y;
+                            y = t;
+                            S* u = px;
+                            px = py;
+                            py = u;
+                            swap = !swap;
+                        }
+                    };
+                    cs(i1, i5, p1, p5);
+                    cs(i2, i4, p2, p4);
+                    cs(i1, i3, p1, p3);
+                    cs(i3, i5, p3, p5);
+                    cs(i1, i2, p1, p2);
+                    cs(i3, i4, p3, p4);
+                    cs(i2, i5, p2, p5);
+                    cs(i2, i3, p2, p3);
+                    cs(i4, i5, p4, p5);
+                    det = (S)-insphere_exact(p1, p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
+                    int depth = 0;
+                    while (det == (S)0) {
+                        ++depth;
+                        if (depth == 1) {
+                            bool c1;
+                            det = orient3d_filter(p2, p3, p4, p5, &c1);
+                            if (!c1) det = (S)orient3d_exact(p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
+                        } else if (depth == 2) {
+                            bool c2;
+                            det = orient3d_filter(p1, p3, p4, p5, &c2);
+                            if (!c2) det = (S)orient3d_exact(p1, p3, p4, p5, ws, (int)kExactWs3D, &over);
+                            det = -det;
+                        } else {
+                            det = swap ? (S)1 : (S)-1;
+                        }
                     }
-                };
-                cs(i1, i5, p1, p5);
-                cs(i2, i4, p2, p4);
-                cs(i1, i3, p1, p3);
-                cs(i3, i5, p3, p5);
-                cs(i1, i2, p1, p2);
-                cs(i3, i4, p3, p4);
-                cs(i2, i5, p2, p5);
-                cs(i2, i3, p2, p3);
-                cs(i4, i5, p4, p5);
-                det = (S)-insphere_exact(p1, p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
-                int depth = 0;
-                while (det == (S)0) {
-                    ++depth;
-                    if (depth == 1) {
-                        bool c1;
-                        det = orient3d_filter(p2, p3, p4, p5, &c1);
-                        if (!c1) det = (S)orient3d_exact(p2, p3, p4, p5, ws, (int)kExactWs3D, &over);
-                    } else if (depth == 2) {
-                        bool c2;
-                        det = orient3d_filter(p1, p3, p4, p5, &c2);
-                        if (!c2) det = (S)orient3d_exact(p1, p3, p4, p5, ws, (int)kExactWs3D, &over);
-                        det = -det;
-                    } else {
-                        det = swap ? (S)1 : (S)-1;
-                    }
+                    if (swap) det = -det;
                 }
-                if (swap) det = -det;
+                wave_lds_sync();
             }
-            if (det > (S)0) {
-                ++Rsize;
-                --Tlast;
-                T(ti) = T(Tlast);
-                T(Tlast) = tl;
-            } else {
-                ++ti;
+            const uint64_t m = __builtin_amdgcn_ballot_w64(det > (S)0);
+            f[0] = q == 0 ? m : f[0];
+            f[1] = q == 1 ? m : f[1];
+            f[2] = q == 2 ? m : f[2];
+            f[3] = q == 3 ? m : f[3];
+        }
+        // the cavity: the sequential order of cpp:421-495 (a conflicting
+        // tetrahedron is swapped with the last one, which is tested next at
+        // the same position)
+        auto flag = [&](uint32_t k) -> bool {
+            const uint64_t w = k < 64 ? f[0] : (k < 128 ? f[1] : (k < 192 ? f[2] : f[3]));
+            return (w >> (k & 63u)) & 1u;
+        };
+        // first flagged position >= k (256 when none)
+        auto next_flag = [&](uint32_t k) -> uint32_t {
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                if (k < q * 64 + 64) {
+                    const uint64_t m = k > q * 64 ? f[q] & (~0ull << (k - q * 64)) : f[q];
+                    if (m) return q * 64 + (uint32_t)__builtin_ctzll(m);
+                }
             }
+            return 256u;
+        };
+        uint32_t Rsize = 0;
+        wave_lds_sync();
+        for (uint32_t ti = next_flag(0); ti < Tlast; ti = next_flag(ti)) {
+            ++Rsize;
+            --Tlast;
+            const uint32_t tl = T(ti), te = T(Tlast);
+            T(ti) = te;
+            T(Tlast) = tl;
+            const bool fl = flag(Tlast);
+            const uint64_t bit = 1ull << (ti & 63u);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if (ti >> 6 == q) f[q] = fl ? f[q] | bit : f[q] & ~bit;
         }
         if (Rsize) {
-            // the star's tetrahedra use local ids below pi only
-            for (uint32_t v = 0; v < pi; ++v) C(v) = (uint8_t)kEmpty;
+            for (uint32_t v = lane; v < kCycle3D; v += 64) C(v) = kEmpty;
+            wave_lds_sync();
             uint32_t first;
-            cavity_walk(T, C, Tlast, Rsize, &first);
+            if (Rsize <= 64)
+                wave_walk(T, C, Tlast, Rsize, &first);
+            else
+                cavity_walk(T, C, Tlast, Rsize, &first);
             uint32_t c = first;
             int guard = 0;
+            bool bad = false;
             do {
-                if (c >= kCycle3D || ++guard > 255 || Tlast >= kTet3D) {
-                    raise_flag(a.flags, kErrCapacity);
-                    break;
-                }
+                bad = c >= kCycle3D || ++guard > 255 || Tlast >= kTet3D;
+                if (bad) break;
                 const uint32_t nx = C(c);
                 T(Tlast++) = pack_tet(pi, c, nx);
                 c = nx;
             } while (c != first);
+            if (bad) {
+                raise_flag(a.flags, kErrCapacity);
+                Tlast = 0;
+                break;
+            }
         }
+        wave_lds_sync();
     }
     if (over) raise_flag(a.flags, kErrCapacity);
-    // alpha filter (cpp:590-682)
-    bool bnd = false;
-    uint32_t nout = 0, nloc = 0;
-    for (uint32_t v = 0; v < ncand; ++v) C(v) = 0;
-    uint32_t ti = 0;
-    while (ti < Tlast) {
-        const uint32_t tl = T(ti);
-        const uint32_t la = tl & 255u, lb = (tl >> 8) & 255u, lc = (tl >> 16) & 255u;
-        bool own = false;
-        const bool inf = la < kNInf3D || lb < kNInf3D || lc < kNInf3D;
-        if (inf || !alpha_keep(P, tid, neig(la), neig(lb), neig(lc), &own)) {
-            bnd = true;
-            --Tlast;
-            T(ti) = T(Tlast);
-            continue;
+    // alpha filter (cpp:590-682): kept tetrahedra count at their corners; this
+    // node's own ones come first, a dropped or foreign one giving its position
+    // to the last one that is left
+    for (uint32_t v = lane; v < ncand; v += 64) C(v) = 0;
+    wave_lds_sync();
+    uint32_t nloc = 0;
+#pragma unroll 1
+    for (uint32_t q = 0; q * 64 < Tlast; ++q) {
+        const uint32_t ti = q * 64 + lane;
+        bool keep = false, own = false;
+        if (ti < Tlast) {
+            const uint32_t tl = T(ti);
+            const uint32_t la = tl & 255u, lb = (tl >> 8) & 255u, lc = (tl >> 16) & 255u;
+            if (la >= kNInf3D && lb >= kNInf3D && lc >= kNInf3D)
+                keep = alpha_keep(P, tid, neig(la), neig(lb), neig(lc), &own);
+            if (keep) {
+                atomicAdd(&C(la), 1u);
+                atomicAdd(&C(lb), 1u);
+                atomicAdd(&C(lc), 1u);
+            }
+            T(ti) = tl | (keep && own ? 1u << 24 : 0u);
         }
-        C(la) = (uint8_t)(C(la) + 1);
-        C(lb) = (uint8_t)(C(lb) + 1);
-        C(lc) = (uint8_t)(C(lc) + 1);
-        ++nloc;
-        if (own) {
-            ++nout;
+        nloc += __popcll(__builtin_amdgcn_ballot_w64(keep));
+    }
+    wave_lds_sync();
+    // per candidate, the number of kept tetrahedra using it (the infinity
+    // nodes are in no kept tetrahedron)
+    uint32_t nf = 0;
+    for (uint32_t v0 = kNInf3D; v0 < ncand; v0 += 64) {
+        const uint32_t v = v0 + lane, c = v < ncand ? C(v) : 0u;
+        if (v < ncand) a.active[slab3(tid, v - kNInf3D, kCand3D)] = (uint8_t)c;
+        nf += __popcll(__builtin_amdgcn_ballot_w64(c != 0));
+    }
+    if (lane != 0) return;
+    uint32_t nout = 0, left = Tlast;
+    for (uint32_t ti = 0; ti < left;) {
+        const uint32_t tl = T(ti);
+        if (tl >> 24) {
+            a.tet[slab3(tid, nout++, kTet3D)] = tl & 0xffffffu;
             ++ti;
         } else {
-            --Tlast;
-            T(ti) = T(Tlast);
+            T(ti) = T(--left);
         }
     }
-    // per candidate, the number of kept tetrahedra using it (counted in
-    // LDS, stored once; the infinity nodes are in no kept tetrahedron)
-    uint32_t nf = 0;
-    for (uint32_t v = kNInf3D; v < ncand; ++v) {
-        const uint8_t c = C(v);
-        a.active[slab3(tid, v - kNInf3D, kCand3D)] = c;
-        nf += c != 0;
-    }
-    a.node_is_bnd[tid] = bnd;
+    a.node_is_bnd[tid] = nloc != Tlast;
     a.nelem_out[tid] = (uint8_t)nout;
     a.nelem[tid] = (uint8_t)nloc;
     a.nfneig[tid] = nf;
@@ -513,12 +598,6 @@ struct Star3Lds {
     uint32_t t[kStarTets];  // ids: removed ones; the whole star for a large cavity
 };
 
-// LDS written by other lanes of this wavefront: program order is execution
-// order there, so only the compiler has to be held.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 __device__ __forceinline__ uint64_t ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }
 // Bits of this lane's group of 16 in a wavefront ballot.
 __device__ __forceinline__ uint32_t group_bits(uint64_t m, uint32_t grp) {
@@ -1061,16 +1140,19 @@ template <class S> void launch_star3(const Ash3Args<S>& a, hipStream_t s) {
     hipLaunchKernelGGL((star3_kernel<S>), dim3(8 * per_xcd), dim3(64), 0, s, a, per_xcd);
 }
 
-// One queued node per wavefront (lane 0; the block is one wavefront): the
-// exact evaluations of different nodes happen at different points of their
+// One queued node per wavefront (the block is one wavefront): the exact
+// evaluations of different nodes happen at different points of their
 // insertions, so nodes sharing a wavefront would run their exact stages one
-// after another.  The expansion workspace lives in LDS.
+// after another.  Bound: the latency of one node's chain.  A single open star
+// that outgrew 64 tetrahedra (tank, 299,000 nodes): 1.94 ms by one lane, star
+// and coordinates in global memory; 0.23 ms by the wavefront, both in LDS.
 template <class S> __global__ __launch_bounds__(64) void delaunay3_exact_kernel(Ash3Args<S> a) {
-    __shared__ uint8_t cyc[kCycle3D];
-    __shared__ double ws[kExactWs3D];
-    if (threadIdx.x != 0) return;
+    __shared__ Exact3Lds<S> lds;
     const uint32_t cnt = a.queue[0];
-    for (uint32_t k = blockIdx.x; k < cnt; k += gridDim.x) local_delaunay3_exact<S>(a, a.queue[kQueueIds + k], cyc, ws);
+    for (uint32_t k = blockIdx.x; k < cnt; k += gridDim.x) {
+        local_delaunay3_exact<S>(a, a.queue[kQueueIds + k], lds);
+        wave_lds_sync();
+    }
 }
 
 // Slab -> CSR (cpp:692-735): edges with count <= 3 are boundary edges; the
@@ -1171,7 +1253,9 @@ template <class S> void Ash3D<S>::compute(hipStream_t s) {
     Ash3Args<S> a = make_args3(*this);
     section_mark(s, kMarkCompute0);
     fill<uint32_t>(queue.p, kQueueIds, 0u, s);
-    hipLaunchKernelGGL((fill3_kernel<S>), dim3(grid_for(n, 256)), dim3(256), 0, s, a);
+    constexpr uint32_t fill_nodes = kFillBlock / kFillLanes3D;
+    const uint32_t fill_xcd = ((n + fill_nodes - 1) / fill_nodes + 7) / 8;
+    hipLaunchKernelGGL((fill3_kernel<S>), dim3(8 * fill_xcd), dim3(kFillBlock), 0, s, a, fill_xcd);
     section_mark(s, kMarkFill);
     launch_star3(a, s);
     section_mark(s, kMarkDelaunayMain);
