@@ -23,7 +23,7 @@ constexpr uint32_t kMsgPart = 256;                   // e_w 192, m_b 64
 constexpr uint32_t kEncPart = (kNodeFeats + 1) * kHid;  // enc_w 5 x 64, enc_b 64
 constexpr uint32_t kEdgeGrid = 2048;                 // blocks of the partial-writing edge kernels
 constexpr uint32_t kGemmGrid = 2048;
-constexpr uint32_t kDwGrid = 512;
+constexpr uint32_t kDwGrid = 1280;
 
 // BF16 [out][in] copies for the forward GEMMs.
 constexpr uint32_t wt_pq(uint32_t l) { return l * 4u * kHid * kHid; }
@@ -904,9 +904,15 @@ GemmArgs gargs(uint32_t n, const float* x0, uint32_t ld0, const uint16_t* wt, fl
 template <int K, int K0, int N, bool BIAS>
 void run_dw(uint32_t n, const float* x0, uint32_t ld0, const float* x1, uint32_t ld1, const float* dy,
             uint32_t lddy, float* partial, float* dst, hipStream_t s) {
-    const uint32_t nb = blocks_for(n, 256, kDwGrid);
-    uint32_t rpb = (n + nb - 1) / nb;
-    rpb = (rpb + 31) / 32 * 32;
+    // Bound: the latency of a block's 32-row stages, so as few of them per block
+    // as kDwGrid allows: 256 rows per block (one block per CU at 65k nodes) took
+    // 87, 67 and 104 us per product, 64 rows 32, 24 and 42 us; small graphs gain
+    // most (a gradient on 2,400 nodes 838 -> 510 us).  Beyond kDwGrid blocks the
+    // partials' traffic costs more (160k nodes: 2.41 ms at 1,000 blocks, 2.52 at
+    // 1,667).
+    uint32_t rpb = (n + kDwGrid - 1) / kDwGrid;
+    rpb = rpb ? (rpb + 31) / 32 * 32 : 32;
+    const uint32_t nb = n ? (n + rpb - 1) / rpb : 1;
     const uint32_t width = K * N + (BIAS ? N : 0);
     hipLaunchKernelGGL((gemm_dw_kernel<K, K0, N, BIAS>), dim3(nb), dim3(256), 0, s, n, rpb, x0, ld0, x1, ld1, dy,
                        lddy, partial);

@@ -25,7 +25,7 @@ def _chain_lattice(n):
     return A.indptr.astype(np.uint32), A.indices.astype(np.uint32), A.data.astype(np.float64), xy, bnd
 
 
-@pytest.mark.parametrize("n", [4, 252, 256, 257, 1024, 1025])
+@pytest.mark.parametrize("n", [4, 32, 33, 252, 256, 257, 1024, 1025, 2049])
 def test_gradient_matches_oracle(n):
     from stream_amd.learned import PrecLearned
 
