@@ -904,8 +904,11 @@ __global__ __launch_bounds__(NT) void cg_update_kernel(uint32_t n, XV* __restric
 // that plain CG solves).  Bound: the launch and the chain entries -> records ->
 // sums, not bytes.  State k lives in record buffer, partials and history k & 1,
 // so that no kernel writes what another block of it still reads; every block
-// derives the same scalars and stop decision from the same partials.  x lags:
-// state k's x is complete once kernel k has run.
+// derives the same scalars and stop decision from the same partials.  The stop
+// is part of the history for that reason: a wavefront that saw a flag raised by
+// its own launch would leave the others of its block with half a sum, and x
+// with a step of garbage.  Kernel k adds alpha_k p_k to x, so state k's x is
+// complete before it runs.
 template <class V> struct alignas(4 * sizeof(V)) CgRec {
     V u, us, p, pad;
 };
@@ -933,7 +936,6 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
                                                  const CgRec<V>* __restrict__ cur, CgRec<V>* __restrict__ nxt,
                                                  double* __restrict__ x, CgScalars* sc, Cg1Hist* hist,
                                                  double* partials, uint32_t par) {
-    const uint32_t done = flag_load(&sc->done);
     const Cg1Hist h = hist[par];
     const double* pin = partials + kCg1Slot + (size_t)par * 5 * kMaxCgBlocks;
     const auto pf = prefetch_partials<5, NT, kCg1Prefetch>(pin, kMaxCgBlocks, gridDim.x);
@@ -952,10 +954,13 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
         for (int q = 0; q < CH; ++q) g[q] = cg1_load(cur, c[q]);
     };
     load(0);
-    if (done) return;
+    const bool first_thread = blockIdx.x == 0 && threadIdx.x == 0;
+    if (h.done) {
+        if (first_thread) hist[par ^ 1u] = h;
+        return;
+    }
     double tot[5];
     sum_prefetched<5, NT, kCg1Prefetch>(pf, pin, kMaxCgBlocks, gridDim.x, tot);
-    const bool first_thread = blockIdx.x == 0 && threadIdx.x == 0;
     // FP32 vectors: the recursion goes on to 0.6 of the tolerance (3% more
     // iterations at 1e-8), so that the true residual, which its rounding moves
     // by several percent, meets the tolerance at the first look
@@ -965,7 +970,8 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
         if (first_thread) {
             sc->rr = tot[4];
             sc->rz = tot[0];
-            sc->done = 1u;
+            sc->done = 1u;  // for the host
+            hist[par ^ 1u] = {h.iter, 0u, 1u, 0u};
         }
         return;
     }
@@ -973,7 +979,7 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
     const double nu = tot[0] - 2.0 * alpha * tot[2] + alpha * alpha * tot[3];
     const double beta = fmax(nu, 0.0) / tot[0];
     if (first_thread) {
-        hist[par ^ 1u] = {h.iter + 1, 0u};
+        hist[par ^ 1u] = {h.iter + 1, 0u, 0u, 0u};
         sc->rr = tot[4];
         sc->rz = tot[0];
         sc->alpha = alpha;
@@ -1029,6 +1035,7 @@ __global__ __launch_bounds__(NT) void cg1_start_kernel(uint32_t n, const V* __re
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (!replaced) hist[par].iter = 0u;
         hist[par].fresh = 1u;
+        hist[par].done = 0u;
     }
 }
 // s = A p of that state (in place: only p is read from other rows) and its

@@ -101,6 +101,8 @@ struct CgScalars {
 struct Cg1Hist {
     uint32_t iter;   // k
     uint32_t fresh;  // the residual kernel tested this state already
+    uint32_t done;   // an earlier kernel stopped at state `iter`: do nothing, pass it on
+    uint32_t pad;
 };
 
 struct CgWork {

@@ -1,7 +1,7 @@
 """The one-kernel Jacobi-PCG iteration at the edges of its rule: row counts
 around a wavefront, a block, the 256 / 512 thread blocks and the two-kernel
 iteration, rows from empty to wider than one load step, a starting guess, the
-iteration cap, and graph replay.  Oracle: textbook FP64 PCG and the FP64
+iteration cap, a stop inside a batch of launches, and graph replay.  Oracle: textbook FP64 PCG and the FP64
 residual b - A x, both in numpy / scipy."""
 import numpy as np
 import pytest
@@ -118,5 +118,30 @@ def test_graph_replay_gives_the_same_bits():
         finally:
             tune("graph", 0)
         xs.append(x)
+    for x in xs[1:]:
+        assert np.array_equal(x, xs[0])
+
+
+@pytest.mark.parametrize("n", [3_000, 65_536, 65_537, 131_072])
+def test_launches_behind_the_stop_change_nothing(n):
+    """The stop falls on the last launch of a batch or has up to 63 launches
+    behind it: the same iterations and the same bits either way."""
+    from stream_amd import tune
+    from stream_amd.numerics import SolverCG
+
+    print(f"[cg one] stop n={n}", flush=True)
+    A = _band(n, 3)
+    b = np.random.default_rng(11).standard_normal(n)
+    s, prec = _system(A, b)
+    its, xs = [], []
+    for batch in (1, 2, 7, 32, 33, 64):
+        tune("batch", batch)
+        try:
+            x = np.zeros(n)
+            its.append(SolverCG().solve_rel(s, prec, x, rtol=1e-9)[0])
+        finally:
+            tune("batch", 32)
+        xs.append(x)
+    assert len(set(its)) == 1
     for x in xs[1:]:
         assert np.array_equal(x, xs[0])
