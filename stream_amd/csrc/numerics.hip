@@ -909,6 +909,12 @@ __global__ __launch_bounds__(NT) void cg_update_kernel(uint32_t n, XV* __restric
 // its own launch would leave the others of its block with half a sum, and x
 // with a step of garbage.  Kernel k adds alpha_k p_k to x, so state k's x is
 // complete before it runs.
+// The rounding of r, u and alpha to V and of the products behind the sums moves
+// the next nu by at most 8 u (nu + alpha^2 gamma), u = half an ulp of 1.  Within
+// twice that (kCg1Noise) beta is taken as 0: the true one is then below 2e-6 in
+// FP32, and beta p under a few thousandths of u.  A diagonal system, which is
+// solved in one step but for rounding, would otherwise leave its solution again
+// along a beta of pure rounding.
 template <class V> struct alignas(4 * sizeof(V)) CgRec {
     V u, us, p, pad;
 };
@@ -930,6 +936,7 @@ __device__ __forceinline__ void cg1_sums(double (&v)[5], V u, V us, V p, V acc, 
     v[4] += r * r;
 }
 
+template <class V> constexpr double kCg1Noise = sizeof(V) == 4 ? 0x1p-20 : 0x1p-49;  // 16 u
 constexpr int kCg1Prefetch = 8;  // 5 x G partials, G <= 409 blocks of 256 or 819 of 512
 template <class V, bool DIFF, int PREC, int CH, int NT>
 __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restrict__ idiag,
@@ -977,7 +984,7 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
     }
     const double alpha = tot[0] / tot[1];
     const double nu = tot[0] - 2.0 * alpha * tot[2] + alpha * alpha * tot[3];
-    const double beta = fmax(nu, 0.0) / tot[0];
+    const double beta = nu > kCg1Noise<V> * (tot[0] + alpha * alpha * tot[3]) ? nu / tot[0] : 0.0;
     if (first_thread) {
         hist[par ^ 1u] = {h.iter + 1, 0u, 0u, 0u};
         sc->rr = tot[4];

@@ -1,7 +1,8 @@
 """The one-kernel Jacobi-PCG iteration at the edges of its rule: row counts
 around a wavefront, a block, the 256 / 512 thread blocks and the two-kernel
 iteration, rows from empty to wider than one load step, a starting guess, the
-iteration cap, a stop inside a batch of launches, and graph replay.  Oracle: textbook FP64 PCG and the FP64
+iteration cap, a stop inside a batch of launches, systems that one step solves,
+and graph replay.  Oracle: textbook FP64 PCG and the FP64
 residual b - A x, both in numpy / scipy."""
 import numpy as np
 import pytest
@@ -145,3 +146,21 @@ def test_launches_behind_the_stop_change_nothing(n):
     assert len(set(its)) == 1
     for x in xs[1:]:
         assert np.array_equal(x, xs[0])
+
+
+@pytest.mark.parametrize("n", [1, 2, 65, 3_000])
+def test_systems_that_one_step_solves(n):
+    """Diagonal systems: all that is left after a step is rounding, 1e-14 of r.z
+    in FP32.  Every step then brings six or seven digits of the 1e-10, so 3 do."""
+    from stream_amd.numerics import SolverCG
+
+    print(f"[cg one] diagonal n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    for _ in range(20 if n < 3 else 3):
+        A = sp.diags(0.1 + 4.0 * rng.random(n)).tocsr()
+        b = rng.standard_normal(n)
+        s, prec = _system(A, b)
+        for solve in (SolverCG().solve_mixed, SolverCG().solve_rel):
+            x = np.zeros(n)
+            it, _ = solve(s, prec, x, rtol=1e-10, maxit=100)
+            assert it <= 3 and _rel(A, b, x) <= 1e-10 * (1 + 1e-6)
