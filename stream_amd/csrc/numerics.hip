@@ -911,7 +911,7 @@ __global__ __launch_bounds__(NT) void cg_update_kernel(uint32_t n, XV* __restric
 // complete before it runs.
 // The rounding of r, u and alpha to V and of the products behind the sums moves
 // the next nu by at most 8 u (nu + alpha^2 gamma), u = half an ulp of 1.  Within
-// twice that (kCg1Noise) beta is taken as 0: the true one is then below 2e-6 in
+// twice that (kCg1Noise; both sides change sign with A) beta is taken as 0: the true one is then below 2e-6 in
 // FP32, and beta p under a few thousandths of u.  A diagonal system, which is
 // solved in one step but for rounding, would otherwise leave its solution again
 // along a beta of pure rounding.
@@ -984,7 +984,8 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
     }
     const double alpha = tot[0] / tot[1];
     const double nu = tot[0] - 2.0 * alpha * tot[2] + alpha * alpha * tot[3];
-    const double beta = nu > kCg1Noise<V> * (tot[0] + alpha * alpha * tot[3]) ? nu / tot[0] : 0.0;
+    const double beta =
+        fabs(nu) > kCg1Noise<V> * (fabs(tot[0]) + alpha * alpha * fabs(tot[3])) ? nu / tot[0] : 0.0;
     if (first_thread) {
         hist[par ^ 1u] = {h.iter + 1, 0u, 0u, 0u};
         sc->rr = tot[4];

@@ -2,7 +2,7 @@
 around a wavefront, a block, the 256 / 512 thread blocks and the two-kernel
 iteration, rows from empty to wider than one load step, a starting guess, the
 iteration cap, a stop inside a batch of launches, systems that one step solves,
-and graph replay.  Oracle: textbook FP64 PCG and the FP64
+negative definite ones, and graph replay.  Oracle: textbook FP64 PCG and the FP64
 residual b - A x, both in numpy / scipy."""
 import numpy as np
 import pytest
@@ -164,3 +164,21 @@ def test_systems_that_one_step_solves(n):
             x = np.zeros(n)
             it, _ = solve(s, prec, x, rtol=1e-10, maxit=100)
             assert it <= 3 and _rel(A, b, x) <= 1e-10 * (1 + 1e-6)
+
+
+@pytest.mark.parametrize("mixed, n", [(False, 3_600), (False, 131_072), (False, 131_073), (True, 3_600),
+                                      (True, 196_608), (True, 196_609)])
+def test_negative_definite_systems(n, mixed):
+    """-A with its own diagonal: the iterates of A, every scalar product negated."""
+    from stream_amd.numerics import SolverCG
+
+    print(f"[cg one] negative n={n} mixed={mixed}", flush=True)
+    A = _band(n, 3)
+    b = np.random.default_rng(23).standard_normal(n)
+    its = []
+    for sign in (1.0, -1.0):
+        s, prec = _system(sign * A, b)
+        x = np.zeros(n)
+        its.append((SolverCG().solve_mixed if mixed else SolverCG().solve_rel)(s, prec, x, rtol=1e-8, maxit=2000)[0])
+        assert _rel(sign * A, b, x) <= 1e-8 * (1 + 1e-6)
+    assert its[0] == its[1]
