@@ -891,58 +891,58 @@ __global__ __launch_bounds__(NT) void cg_update_kernel(uint32_t n, XV* __restric
 // predict-and-recompute CG (T. Chen and E. Carson, "Predict-and-Recompute
 // Conjugate Gradient Variants", SIAM J. Sci. Comput. 42, 2020).  With u =
 // M^-1 r and s = A p, every scalar comes from sums that one pass over the
-// vectors of a state gives, nu = u.r, mu = p.s, delta = u.s and gamma = s.M^-1 s:
+// vectors of a state gives, nu = r.u, mu = p.s, delta = u.s and gamma = s.M^-1 s:
 //   alpha = nu / mu, beta = (nu - 2 alpha delta + alpha^2 gamma) / nu
 // (the numerator is the next nu, expanded; alpha uses the recomputed one), then
-//   x += alpha p, u -= alpha M^-1 s, p = u + beta p, s = A p.
+//   x += alpha p, r -= alpha s, u = M^-1 r, p = u + beta p, s = A p.
 // cg_dir / cg_update wait for the grid twice per iteration.  Here a row forms
-// its neighbours' new p itself from one record {u, M^-1 s, p} each (their
+// its neighbours' new p itself from one record {r, s, p, M^-1} each (their
 // owners' operations, so the same bits), and the grid is waited for once,
-// between launches.  s is a product in every iteration, as in plain CG, so
-// the residual drifts no faster: iteration counts are the two-kernel ones' to
-// a few in a thousand (forms with a recursion for s failed on FP32 systems
-// that plain CG solves).  Bound: the launch and the chain entries -> records ->
-// sums, not bytes.  State k lives in record buffer, partials and history k & 1,
-// so that no kernel writes what another block of it still reads; every block
-// derives the same scalars and stop decision from the same partials.  The stop
-// is part of the history for that reason: a wavefront that saw a flag raised by
-// its own launch would leave the others of its block with half a sum, and x
-// with a step of garbage.  Kernel k adds alpha_k p_k to x, so state k's x is
-// complete before it runs.
+// between launches.  The record holds r, and M^-1 beside it, and not u: r
+// cannot be had back from u, since M need not be the system's own diagonal and
+// an entry of M^-1 may be 0 in this precision.  s is a product in every
+// iteration, as in plain CG, so the residual drifts no faster: iteration counts
+// are the two-kernel ones' to a few in a thousand (forms with a recursion for s
+// failed on FP32 systems that plain CG solves).  Bound: the launch and the chain
+// entries -> records -> sums, not bytes.
+// State k lives in record buffer, partials and history k & 1, so that no kernel
+// writes what another block of it still reads; every block derives the same
+// scalars and stop decision from the same partials.  The stop is part of the
+// history for that reason: a wavefront that saw a flag raised by its own launch
+// would leave the others of its block with half a sum, and x with a step of
+// garbage.  Kernel k adds alpha_k p_k to x, so state k's x is complete before it
+// runs.
 // The rounding of r, u and alpha to V and of the products behind the sums moves
-// the next nu by at most 8 u (nu + alpha^2 gamma), u = half an ulp of 1.  Within
-// twice that (kCg1Noise; both sides change sign with A) beta is taken as 0: the true one is then below 2e-6 in
-// FP32, and beta p under a few thousandths of u.  A diagonal system, which is
-// solved in one step but for rounding, would otherwise leave its solution again
-// along a beta of pure rounding.
+// the next nu by at most 8 e (nu + alpha^2 gamma), e = half an ulp of 1.  Within
+// twice that (kCg1Noise; both sides change sign with A) beta is taken as 0: the
+// true one is then below 2e-6 in FP32, and beta p under a few thousandths of u.
+// A diagonal system, which is solved in one step but for rounding, would
+// otherwise leave its solution again along a beta of pure rounding.
 template <class V> struct alignas(4 * sizeof(V)) CgRec {
-    V u, us, p, pad;
+    V r, s, p, m;
 };
-template <class V> struct CgRow {
-    V u, us, p;
-};
-template <class V> __device__ __forceinline__ CgRow<V> cg1_load(const CgRec<V>* rec, uint32_t i) {
-    return {rec[i].u, rec[i].us, rec[i].p};
+// A row's new r and p.
+template <class V> __device__ __forceinline__ V cg1_r(const CgRec<V>& c, V alpha) { return c.r - alpha * c.s; }
+template <class V> __device__ __forceinline__ V cg1_p(const CgRec<V>& c, V alpha, V beta) {
+    return c.m * cg1_r(c, alpha) + beta * c.p;
 }
 
-// The sums of a state, a row's part; acc = (A p)_i, r = u / M^-1.
-template <class V, bool DIFF, int PREC>
-__device__ __forceinline__ void cg1_sums(double (&v)[5], V u, V us, V p, V acc, V diag, V idiag) {
-    const double r = PREC == kPrecNone ? (double)u : (DIFF ? (double)u / (double)idiag : (double)diag * (double)u);
-    v[0] += r * (double)u;
-    v[1] += (double)acc * (double)p;
-    v[2] += (double)acc * (double)u;
-    v[3] += (double)acc * (double)us;
-    v[4] += r * r;
+// The sums of a state, a row's part.
+template <class V> __device__ __forceinline__ void cg1_sums(double (&v)[5], const CgRec<V>& c) {
+    const V u = c.m * c.r;
+    v[0] += (double)c.r * (double)u;
+    v[1] += (double)c.s * (double)c.p;
+    v[2] += (double)c.s * (double)u;
+    v[3] += (double)c.s * (double)(c.m * c.s);
+    v[4] += (double)c.r * (double)c.r;
 }
 
-template <class V> constexpr double kCg1Noise = sizeof(V) == 4 ? 0x1p-20 : 0x1p-49;  // 16 u
+template <class V> constexpr double kCg1Noise = sizeof(V) == 4 ? 0x1p-20 : 0x1p-49;  // 16 e
 constexpr int kCg1Prefetch = 8;  // 5 x G partials, G <= 409 blocks of 256 or 819 of 512
-template <class V, bool DIFF, int PREC, int CH, int NT>
-__global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restrict__ idiag,
-                                                 const CgRec<V>* __restrict__ cur, CgRec<V>* __restrict__ nxt,
-                                                 double* __restrict__ x, CgScalars* sc, Cg1Hist* hist,
-                                                 double* partials, uint32_t par) {
+template <class V, bool DIFF, int CH, int NT>
+__global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const CgRec<V>* __restrict__ cur,
+                                                 CgRec<V>* __restrict__ nxt, double* __restrict__ x, CgScalars* sc,
+                                                 Cg1Hist* hist, double* partials, uint32_t par) {
     const Cg1Hist h = hist[par];
     const double* pin = partials + kCg1Slot + (size_t)par * 5 * kMaxCgBlocks;
     const auto pf = prefetch_partials<5, NT, kCg1Prefetch>(pin, kMaxCgBlocks, gridDim.x);
@@ -951,14 +951,14 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
     // the first slice's own records, entries and gathers before the sum
     SliceRows<1> rows = slice_rows<V, 1>(M, sp.s, sp, lane);
     uint32_t seg = rows.base[0];
-    CgRow<V> own = cg1_load(cur, rows.ii[0]);
+    CgRec<V> own = cur[rows.ii[0]];
     V a[CH];
-    CgRow<V> g[CH];
+    CgRec<V> g[CH];
     auto load = [&](uint32_t k) {
         uint32_t c[CH];
         sell_load<V, CH>(M, seg, k, rows.L[0], rows.ii[0], c, a);
 #pragma unroll
-        for (int q = 0; q < CH; ++q) g[q] = cg1_load(cur, c[q]);
+        for (int q = 0; q < CH; ++q) g[q] = cur[c[q]];
     };
     load(0);
     const bool first_thread = blockIdx.x == 0 && threadIdx.x == 0;
@@ -998,47 +998,47 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const V* __restr
     double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     for (uint32_t s0 = sp.s;;) {
         const uint32_t i = rows.ii[0];
-        const V un = own.u - av * own.us, pn = un + bv * own.p, dg = M.diag[i];
-        V acc = dg * pn;
+        CgRec<V> st = own;  // the new state
+        st.r = cg1_r(own, av);
+        st.p = cg1_p(own, av, bv);
+        V acc = M.diag[i] * st.p;
         for (uint32_t k = 0;;) {
 #pragma unroll
             for (int q = 0; q < CH; ++q) {
-                const V pj = (g[q].u - av * g[q].us) + bv * g[q].p;
-                acc = DIFF ? acc + a[q] * (pj - pn) : acc + a[q] * pj;
+                const V pj = cg1_p(g[q], av, bv);
+                acc = DIFF ? acc + a[q] * (pj - st.p) : acc + a[q] * pj;
             }
             k += CH;
             if (k >= rows.W) break;
             load(k);
         }
         if (rows.valid[0]) {
-            const V id = PREC == kPrecJacobi ? idiag[i] : (V)1;
-            const V us = id * acc;
-            nxt[i].u = un;
-            nxt[i].us = us;
-            nxt[i].p = pn;
+            st.s = acc;
+            nxt[i] = st;
             x[i] += alpha * (double)own.p;
-            cg1_sums<V, DIFF, PREC>(v, un, us, pn, acc, dg, id);
+            cg1_sums(v, st);
         }
         s0 += sp.step;
         if (s0 >= sp.e) break;
         rows = slice_rows<V, 1>(M, s0, sp, lane);
         seg = rows.base[0];
-        own = cg1_load(cur, rows.ii[0]);
+        own = cur[rows.ii[0]];
         load(0);
     }
     store_partials<5, NT>(v, partials + kCg1Slot + (size_t)(par ^ 1u) * 5 * kMaxCgBlocks, kMaxCgBlocks);
 }
 
-// The state behind a residual kernel (r given): u = M^-1 r, and p = u at the
-// start; a replacement keeps the direction and beta, p += u - u_old.
+// The state behind a residual kernel (r given): p = u = M^-1 r at the start; a
+// replacement keeps the direction and beta, p += u - u_old.
 template <class V, int PREC, int NT>
 __global__ __launch_bounds__(NT) void cg1_start_kernel(uint32_t n, const V* __restrict__ idiag,
                                                        const V* __restrict__ r, CgRec<V>* __restrict__ rec,
                                                        Cg1Hist* hist, uint32_t par, bool replaced) {
     CG_ROWS(i) {
-        const V un = PREC == kPrecJacobi ? idiag[i] * r[i] : r[i];
-        rec[i].p = replaced ? rec[i].p + (un - rec[i].u) : un;
-        rec[i].u = un;
+        const V m = PREC == kPrecJacobi ? idiag[i] : (V)1, rn = r[i], un = m * rn;
+        rec[i].p = replaced ? rec[i].p + (un - m * rec[i].r) : un;
+        rec[i].r = rn;
+        rec[i].m = m;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (!replaced) hist[par].iter = 0u;
@@ -1048,23 +1048,21 @@ __global__ __launch_bounds__(NT) void cg1_start_kernel(uint32_t n, const V* __re
 }
 // s = A p of that state (in place: only p is read from other rows) and its
 // sums.
-template <class V, bool DIFF, int PREC, int CH, int NT>
-__global__ __launch_bounds__(NT) void cg1_apply_kernel(SellArgs<V> M, const V* __restrict__ idiag, CgRec<V>* rec,
-                                                       double* partials, uint32_t par) {
+template <class V, bool DIFF, int CH, int NT>
+__global__ __launch_bounds__(NT) void cg1_apply_kernel(SellArgs<V> M, CgRec<V>* rec, double* partials, uint32_t par) {
     const uint32_t lane = threadIdx.x & 63u;
     double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     SELL_FOR_SLICE_ROWS(1, rows) {
         const uint32_t i = rows.ii[0];
-        const V pn = rec[i].p, dg = M.diag[i];
-        V acc[1] = {dg * pn};
+        CgRec<V> st = rec[i];
+        V acc[1] = {M.diag[i] * st.p};
         sell_rows_product<V, 1, CH, V>(
             M, rows, acc, [&](uint32_t j) -> V { return rec[j].p; },
-            [&](int, V ac, V a, V gj) { return DIFF ? ac + a * (gj - pn) : ac + a * gj; });
+            [&](int, V ac, V a, V gj) { return DIFF ? ac + a * (gj - st.p) : ac + a * gj; });
         if (rows.valid[0]) {
-            const V id = PREC == kPrecJacobi ? idiag[i] : (V)1;
-            const V us = id * acc[0];
-            rec[i].us = us;
-            cg1_sums<V, DIFF, PREC>(v, rec[i].u, us, pn, acc[0], dg, id);
+            st.s = acc[0];
+            rec[i].s = st.s;
+            cg1_sums(v, st);
         }
     }
     store_partials<5, NT>(v, partials + kCg1Slot + (size_t)par * 5 * kMaxCgBlocks, kMaxCgBlocks);
@@ -1368,7 +1366,7 @@ void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const
             residual_kernel(vv.r, 1u, reinterpret_cast<V2<V>*>(vv.D[0]), mode);
             hipLaunchKernelGGL((cg1_start_kernel<V, PREC, NT>), grid, blk, 0, s, n, idiag, vv.r, rec[it & 1],
                                w.hist.p, it & 1u, mode != 0);
-            hipLaunchKernelGGL((cg1_apply_kernel<V, DIFF, PREC, CH, NT>), grid, blk, 0, s, MA, idiag, rec[it & 1],
+            hipLaunchKernelGGL((cg1_apply_kernel<V, DIFF, CH, NT>), grid, blk, 0, s, MA, rec[it & 1],
                                w.partials.p, it & 1u);
             return;
         }
@@ -1389,8 +1387,8 @@ void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const
         for (uint32_t k = 0; k < o.batch; ++k) {
             const uint32_t it = it0 + k;
             if constexpr (ONE) {
-                hipLaunchKernelGGL((cg1_kernel<V, DIFF, PREC, CH, NT>), grid, blk, 0, s, MA, idiag, rec[it & 1],
-                                   rec[(it + 1) & 1], xacc, w.sc.p, w.hist.p, w.partials.p, it & 1u);
+                hipLaunchKernelGGL((cg1_kernel<V, DIFF, CH, NT>), grid, blk, 0, s, MA, rec[it & 1], rec[(it + 1) & 1],
+                                   xacc, w.sc.p, w.hist.p, w.partials.p, it & 1u);
                 continue;
             }
             V2<V>* cur = vv.P[it & 1];
