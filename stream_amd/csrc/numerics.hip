@@ -1509,17 +1509,27 @@ void cg_solve_llt(const DevCsr<double>& A64, const Sell<V>& S, const LowerFactor
         cg_drive<V, DIFF, kPrecLLt, CH, 1, 1024>(A64, S, nullptr, L, b, x, o, w, st, s);
 }
 
-// Block size of the one-kernel iteration of values V on n rows (0: the
-// two-kernel one).  us per iteration, two kernels -> one, FP64: 2D 11.9 -> 7.6
-// (16k rows), 12.1 -> 8.3 (60k), 13.7 -> 9.9 (90k), 14.1 -> 10.7 (130k), 14.9
-// -> 17.5 (150k); 3D 15.0 -> 12.0 (30k), 18.1 -> 17.1 (120k), 23.8 -> 30.2
+// Block size of the one-kernel iteration of values V on n rows with nnz entries
+// (0: the two-kernel one).  us per iteration, two kernels -> one, FP64: 2D 11.9
+// -> 7.6 (16k rows), 12.1 -> 8.3 (60k), 13.7 -> 9.9 (90k), 14.1 -> 10.7 (130k),
+// 14.9 -> 17.5 (150k); 3D 15.0 -> 12.0 (30k), 18.1 -> 17.1 (120k), 23.8 -> 30.2
 // (200k).  FP32: 2D 12.3 -> 7.9 (60k), 13.9 -> 11.7 (150k), 3D 17.6 -> 14.1
 // (120k), 19.8 -> 18.3 (200k), 23.8 -> 28.1 (300k).  The line is where CUs get a
 // second block (FP64: 32-byte records, 12 wavefronts per CU) or where the
 // records' gathers cost more than the second launch.  One block per CU as
 // far as 256 threads allow that: 7.2 against 8.2 us with 512 at 16k.
-template <class V> uint32_t cg1_threads(uint32_t n) {
-    if (n > (sizeof(V) == 8 ? 256u : 384u) * 512u) return 0;
+// A gather of an entry moves twice the bytes, so wide rows lose what the launch
+// saves.  Lattices in Morton order, 96 iterations with start and end, two
+// kernels -> one.  FP64 at 64k rows: 26 entries per row 17.8 -> 16.6, 54 23.6 ->
+// 23.9, 113 38.2 -> 39.5; at 91k: 11 15.7 -> 14.8, 26 20.7 -> 21.3, 54 27.1 ->
+// 31.7, 182 64.4 -> 84.2.  FP32 at 91k: 26 19.4 -> 16.9, 76 30.4 -> 29.4, 114
+// 39.1 -> 37.5, 182 55.6 -> 55.4; at 195k: 11 17.5 -> 17.2, 26 23.0 -> 23.0, 55
+// 29.7 -> 31.6, 186 75.5 -> 94.9.
+template <class V> uint32_t cg1_threads(uint32_t n, uint32_t nnz) {
+    constexpr bool wide = sizeof(V) == 8;
+    if (n > (wide ? 256u : 384u) * 512u) return 0;
+    const uint32_t most = wide ? (n <= 65536u ? 40u : 20u) : (n <= 131072u ? 100u : 20u);
+    if (nnz > (uint64_t)most * n) return 0;
     return n <= 256u * 256u ? 256 : 512;
 }
 
@@ -1540,7 +1550,7 @@ void cg_solve_ch(const DevCsr<double>& A64, const Sell<V>& S, bool diff, int32_t
         constexpr int P = decltype(p)::value;
         // (without the true residual's verdict the result is the recursion's
         // own: those callers keep the two-kernel one)
-        const uint32_t one = o.verify ? cg1_threads<V>(A64.n) : 0u;
+        const uint32_t one = o.verify ? cg1_threads<V>(A64.n, A64.nnz) : 0u;
         if (one == 256)
             cg_drive<V, D, P, CH, 1, 256, true>(A64, S, idiag, L, b, x, o, w, st, s);
         else if (one == 512)

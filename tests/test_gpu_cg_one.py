@@ -1,10 +1,10 @@
 """The one-kernel Jacobi-PCG iteration at the edges of its rule: row counts
 around a wavefront, a block, the 256 / 512 thread blocks and the two-kernel
-iteration, rows from empty to wider than one load step, a starting guess, the
-iteration cap, a stop inside a batch of launches, systems that one step solves,
-negative definite ones, preconditioners that are not the system's own diagonal,
-and graph replay.  Oracle: textbook FP64 PCG and the FP64
-residual b - A x, both in numpy / scipy."""
+iteration, rows from empty to wider than one load step, row widths at the rule's
+lines, a starting guess, the iteration cap, a stop inside a batch of launches,
+systems that one step solves, negative definite ones, preconditioners that are
+not the system's own diagonal, and graph replay.  Oracle: textbook FP64 PCG and
+the FP64 residual b - A x, both in numpy / scipy."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -269,3 +269,27 @@ def test_preconditioner_of_another_matrix(n, mixed, other):
     # back (the two-kernel iteration takes 62 here where FP64 takes 51), and the
     # stop at 0.6 of the tolerance adds 3
     assert abs(it - ref) <= (2 if not mixed else 3 + ref // 4)
+
+
+@pytest.mark.parametrize("n, width, mixed", [(2_000, 27, False), (2_000, 29, False), (70_000, 13, False),
+                                             (70_000, 14, False), (2_000, 69, True), (2_000, 74, True),
+                                             (140_000, 13, True), (140_000, 14, True)])
+def test_both_sides_of_the_row_width_rule(n, width, mixed):
+    """Means of 38.4 and 41.2 (FP64) or 96 and 103 entries per row (FP32), and of
+    19.2 and 20.6 for the larger systems of either."""
+    from stream_amd.numerics import SolverCG
+
+    print(f"[cg one] n={n} width={width} mixed={mixed}", flush=True)
+    A = _band(n, width)
+    b = np.random.default_rng(29).standard_normal(n)
+    s, prec = _system(A, b)
+    x = np.zeros(n)
+    # FP32 at 1e-6, where its rounding costs no iterations yet (at 1e-8 the
+    # two-kernel iteration takes 87 where FP64 takes 50)
+    tol = 1e-6 if mixed else 1e-8
+    it, _ = (SolverCG().solve_mixed if mixed else SolverCG().solve_rel)(s, prec, x, rtol=tol, maxit=2000)
+    ref = _pcg(A, 1.0 / A.diagonal(), b, tol)
+    print(f"[cg one]   {it} iterations, oracle {ref}", flush=True)
+    assert _rel(A, b, x) <= tol * (1 + 1e-6)
+    # (the stop at 0.6 of the tolerance: half a digit, a twentieth of these)
+    assert abs(it - ref) <= (2 if not mixed else 3 + ref // 20)
