@@ -887,7 +887,7 @@ __global__ __launch_bounds__(NT) void cg_update_kernel(uint32_t n, XV* __restric
     }
 }
 
-// One iteration in one kernel, for the Jacobi and the unpreconditioned solver:
+// One iteration in one kernel, for the Jacobi-preconditioned solver:
 // predict-and-recompute CG (T. Chen and E. Carson, "Predict-and-Recompute
 // Conjugate Gradient Variants", SIAM J. Sci. Comput. 42, 2020).  With u =
 // M^-1 r and s = A p, every scalar comes from sums that one pass over the
@@ -1030,12 +1030,12 @@ __global__ __launch_bounds__(NT) void cg1_kernel(SellArgs<V> M, const CgRec<V>* 
 
 // The state behind a residual kernel (r given): p = u = M^-1 r at the start; a
 // replacement keeps the direction and beta, p += u - u_old.
-template <class V, int PREC, int NT>
+template <class V, int NT>
 __global__ __launch_bounds__(NT) void cg1_start_kernel(uint32_t n, const V* __restrict__ idiag,
                                                        const V* __restrict__ r, CgRec<V>* __restrict__ rec,
                                                        Cg1Hist* hist, uint32_t par, bool replaced) {
     CG_ROWS(i) {
-        const V m = PREC == kPrecJacobi ? idiag[i] : (V)1, rn = r[i], un = m * rn;
+        const V m = idiag[i], rn = r[i], un = m * rn;
         rec[i].p = replaced ? rec[i].p + (un - m * rec[i].r) : un;
         rec[i].r = rn;
         rec[i].m = m;
@@ -1364,13 +1364,11 @@ void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const
         V2<V>* cur = vv.P[it & 1];
         if constexpr (ONE) {
             residual_kernel(vv.r, 1u, reinterpret_cast<V2<V>*>(vv.D[0]), mode);
-            hipLaunchKernelGGL((cg1_start_kernel<V, PREC, NT>), grid, blk, 0, s, n, idiag, vv.r, rec[it & 1],
+            hipLaunchKernelGGL((cg1_start_kernel<V, NT>), grid, blk, 0, s, n, idiag, vv.r, rec[it & 1],
                                w.hist.p, it & 1u, mode != 0);
             hipLaunchKernelGGL((cg1_apply_kernel<V, DIFF, CH, NT>), grid, blk, 0, s, MA, rec[it & 1],
                                w.partials.p, it & 1u);
-            return;
-        }
-        if constexpr (PREC == kPrecLLt) {
+        } else if constexpr (PREC == kPrecLLt) {
             V2<V>* rqc = vv.RQ[it & 1];
             residual_kernel(reinterpret_cast<V*>(rqc), 2u, cur, mode);
             hipLaunchKernelGGL((llt_update_kernel<V, XV, CH, R, NT>), grid, blk, 0, s, MU, xacc, vv.D[it & 1], rqc, rqc,
@@ -1389,11 +1387,7 @@ void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const
             if constexpr (ONE) {
                 hipLaunchKernelGGL((cg1_kernel<V, DIFF, CH, NT>), grid, blk, 0, s, MA, rec[it & 1], rec[(it + 1) & 1],
                                    xacc, w.sc.p, w.hist.p, w.partials.p, it & 1u);
-                continue;
-            }
-            V2<V>* cur = vv.P[it & 1];
-            V2<V>* nxt = vv.P[(it + 1) & 1];
-            if constexpr (PREC == kPrecLLt) {
+            } else if constexpr (PREC == kPrecLLt) {
                 V2<V>* rqc = vv.RQ[it & 1];
                 V2<V>* rqn = vv.RQ[(it + 1) & 1];
                 V* dc = vv.D[it & 1];
@@ -1404,6 +1398,8 @@ void cg_drive(const DevCsr<double>& A64, const Sell<V>& S, const V* idiag, const
                 hipLaunchKernelGGL((llt_lo_kernel<V, CH, R, NT>), grid, blk, 0, s, ML, vv.w, dc, vv.D[(it + 1) & 1], w.sc.p,
                                    w.partials.p, 0);
             } else {
+                V2<V>* cur = vv.P[it & 1];
+                V2<V>* nxt = vv.P[(it + 1) & 1];
                 hipLaunchKernelGGL((cg_dir_kernel<V, DIFF, CH, R, NT>), grid, blk, 0, s, MA, cur, nxt, vv.q, 1u, w.sc.p,
                                    w.partials.p);
                 hipLaunchKernelGGL((cg_update_kernel<V, XV, PREC, NT>), grid, blk, 0, s, n, xacc, vv.r, nxt, vv.q, idiag,
@@ -1545,32 +1541,29 @@ void cg_solve_ch(const DevCsr<double>& A64, const Sell<V>& S, bool diff, int32_t
             cg_solve_llt<V, false, CH>(A64, S, L, b, x, o, w, st, s);
         return;
     }
-    auto go = [&](auto d, auto p) {
+    if (prec == kPrecNone) {
+        if (diff)
+            cg_drive<V, true, kPrecNone, CH, 1, NT>(A64, S, nullptr, L, b, x, o, w, st, s);
+        else
+            cg_drive<V, false, kPrecNone, CH, 1, NT>(A64, S, nullptr, L, b, x, o, w, st, s);
+        return;
+    }
+    auto jacobi = [&](auto d) {
         constexpr bool D = decltype(d)::value;
-        constexpr int P = decltype(p)::value;
         // (without the true residual's verdict the result is the recursion's
         // own: those callers keep the two-kernel one)
         const uint32_t one = o.verify ? cg1_threads<V>(A64.n, A64.nnz) : 0u;
         if (one == 256)
-            cg_drive<V, D, P, CH, 1, 256, true>(A64, S, idiag, L, b, x, o, w, st, s);
+            cg_drive<V, D, kPrecJacobi, CH, 1, 256, true>(A64, S, idiag, L, b, x, o, w, st, s);
         else if (one == 512)
-            cg_drive<V, D, P, CH, 1, 512, true>(A64, S, idiag, L, b, x, o, w, st, s);
+            cg_drive<V, D, kPrecJacobi, CH, 1, 512, true>(A64, S, idiag, L, b, x, o, w, st, s);
         else
-            cg_drive<V, D, P, CH, 1, NT>(A64, S, idiag, L, b, x, o, w, st, s);
+            cg_drive<V, D, kPrecJacobi, CH, 1, NT>(A64, S, idiag, L, b, x, o, w, st, s);
     };
-    using Jac = std::integral_constant<int, kPrecJacobi>;
-    using Non = std::integral_constant<int, kPrecNone>;
-    if (diff) {
-        if (prec == kPrecJacobi)
-            go(std::true_type{}, Jac{});
-        else
-            go(std::true_type{}, Non{});
-    } else {
-        if (prec == kPrecJacobi)
-            go(std::false_type{}, Jac{});
-        else
-            go(std::false_type{}, Non{});
-    }
+    if (diff)
+        jacobi(std::true_type{});
+    else
+        jacobi(std::false_type{});
 }
 
 template <class V>
