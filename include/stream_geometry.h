@@ -97,6 +97,11 @@ int32_t Stream_heap_order(uint32_t n, const uint32_t* idx, const float* cost, ui
  * insphere (3, 5 x 3) by the device exact stage compiled for the host; pts
  * float (fp64 = 0) or double (predicates.hpp:342-1100 semantics) */
 int32_t Stream_exact_sign_host(int32_t kind, int32_t fp64, const void* pts, int32_t* sign);
+/* no reference counterpart (verification hook): the FP32 sphere test of the 3D
+ * alpha-shape compiled for the host; pts = p, b, c, d, e (5 x 3), coordinates
+ * scaled for alpha: 1 / -1 where it certifies that e lies inside / outside the
+ * sphere of (p, b, c, d) (the sign of -insphere), 0 where it certifies nothing */
+int32_t Stream_sphere_sign_host(const double* pts, double alpha, int32_t* sign);
 
 /* stable onesweep radix sort of (u64, u32) pairs over the low `bits` bits */
 int32_t Stream_sort_pairs_u64(uint32_t n, const uint64_t* keys, const uint32_t* vals, uint64_t* keys_out,

@@ -518,19 +518,9 @@ template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, u
 // cache line per lane and load).  Here 16 lanes hold the star: lane l the
 // tetrahedra at positions l, l + 16, ... in registers, the ids also in LDS.
 //
-//   test    With the node as origin, corners b, c, d and the new point e, the
-//           insphere value is e.W - V |e|^2 with W = |b|^2 cxd + |c|^2 dxb +
-//           |d|^2 bxc and V = b.(cxd).  W, V and the factors wp, vp of the
-//           error bound are kept per tetrahedron, so a test is 7 FP32
-//           operations on one LDS read.  Coordinates are relative to the
-//           node, divided by a power of two near alpha and rounded to FP32 in
-//           both node types.  Each monomial sees at most 21 roundings and the
-//           bound takes 24 (kSphBound); the sums of absolute monomials are
-//           bounded by the lengths: a component of |c||x||d| by |c| |d|, so
-//           W's by Q (|b| + |c| + |d|) and V's by sqrt(3) Q, Q = |b| |c| |d|.
-//           kSphFloor covers underflow for coordinates up to kSphRange,
-//           beyond which the point is NaN and certifies nothing.  What FP32
-//           cannot certify goes to the FP64 filter on the node's own
+//   test    The sphere test of predicates.hpp: 7 FP32 operations on one LDS
+//           read and what is kept per tetrahedron, in both node types.  What
+//           it cannot certify goes to the FP64 filter on the node's own
 //           coordinates, and a node where that fails too to the exact kernel.
 //           A certified sign is the exact sign, so all three give the same
 //           decisions.
@@ -572,9 +562,6 @@ template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, u
 constexpr int kStarLanes = 16;
 constexpr uint32_t kStarTets = 64;
 constexpr int kStarSlots = (int)kStarTets / kStarLanes;
-constexpr float kSphBound = 1.7320509f * 24.0f * 5.9604644775390625e-08f;
-constexpr float kSphFloor = 1e-20f;
-constexpr float kSphRange = 1e7f;
 constexpr uint32_t kWalkFree = 14;  // R (R - 1) / 2 <= 100, and R + 2 new ones on 16 lanes
 
 // Candidates of the four nodes of a wavefront together (LDS); a node that does
@@ -582,10 +569,6 @@ constexpr uint32_t kWalkFree = 14;  // R (R - 1) / 2 <= 100, and R + 2 new ones 
 // node are usual; 448 bring a wavefront's LDS to 10 KB, four per SIMD.
 constexpr uint32_t kStarPool = 448;
 
-struct SphReg {
-    float wx, wy, wz, v, wp, vp;
-    uint32_t w;  // ids (pack_tet)
-};
 struct alignas(16) SphRec {
     SphReg r;
     uint32_t pos;  // where it comes from
@@ -648,41 +631,17 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
     auto neig = [&](uint32_t j) -> uint32_t { return j < kNInf3D ? n + j : a.cand[slab3(tid, j - kNInf3D, kCand3D)]; };
     const Sph4<S> self = P[tid];
     {
-        const double r = (double)self.r;
-        const double scale = (r > 0.0 && r < 1e300) ? ldexp(1.0, -ilogb(r)) : 1.0;
+        const double scale = sph_scale((double)self.r);
         for (uint32_t j = sub; j < ncand; j += G) {
             const Sph4<S> q = P[neig(j)];
-            float4 e;
-            e.x = (float)(((double)q.c[0] - (double)self.c[0]) * scale);
-            e.y = (float)(((double)q.c[1] - (double)self.c[1]) * scale);
-            e.z = (float)(((double)q.c[2] - (double)self.c[2]) * scale);
-            if (!(fmaxf(fabsf(e.x), fmaxf(fabsf(e.y), fabsf(e.z))) <= kSphRange)) e.x = NAN;
-            e.w = sqrtf(fmaf(e.x, e.x, fmaf(e.y, e.y, e.z * e.z)));
-            E[j] = e;
+            E[j] = sph_point(((double)q.c[0] - (double)self.c[0]) * scale, ((double)q.c[1] - (double)self.c[1]) * scale,
+                             ((double)q.c[2] - (double)self.c[2]) * scale);
         }
     }
     wave_lds_sync();
     uint32_t Tl = 4;
     SphReg rec[NS];
-    // corners b, c, d (ids w); |c|^2 dxb + |d|^2 bxc = b x (|d|^2 c - |c|^2 d)
-    auto make_rec = [&](uint32_t w, const float4& b, const float4& c, const float4& d) {
-        const float x = fmaf(c.y, d.z, -(c.z * d.y)), y = fmaf(c.z, d.x, -(c.x * d.z)),
-                    z = fmaf(c.x, d.y, -(c.y * d.x));
-        const float bb = b.w * b.w, cc = c.w * c.w, dd = d.w * d.w;
-        const float gx = fmaf(dd, c.x, -(cc * d.x)), gy = fmaf(dd, c.y, -(cc * d.y)), gz = fmaf(dd, c.z, -(cc * d.z));
-        const float q = kSphBound * (b.w * c.w) * d.w;
-        SphReg r;
-        r.wx = fmaf(bb, x, fmaf(b.y, gz, -(b.z * gy)));
-        r.wy = fmaf(bb, y, fmaf(b.z, gx, -(b.x * gz)));
-        r.wz = fmaf(bb, z, fmaf(b.x, gy, -(b.y * gx)));
-        r.v = fmaf(b.x, x, fmaf(b.y, y, b.z * z));
-        // sum |e_k| <= sqrt(3) |e|
-        r.wp = q * (b.w + c.w + d.w);
-        r.vp = q;
-        r.w = w;
-        return r;
-    };
-    auto load_rec = [&](uint32_t w) { return make_rec(w, E[w & 255u], E[(w >> 8) & 255u], E[(w >> 16) & 255u]); };
+    auto load_rec = [&](uint32_t w) { return sph_rec(w, E[w & 255u], E[(w >> 8) & 255u], E[(w >> 16) & 255u]); };
     if (sub < 4) {
         const uint32_t w = sub == 0   ? pack_tet(0, 2, 1)
                            : sub == 1 ? pack_tet(1, 2, 3)
@@ -710,9 +669,8 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
         uint64_t in_m[NS];
         bool un[NS];
         auto test = [&](int s) {
-            const SphReg& r = rec[s];
-            const float det = fmaf(e.x, r.wx, fmaf(e.y, r.wy, fmaf(e.z, r.wz, -(ee * r.v))));
-            const float err = fmaf(r.wp, e.w, fmaf(r.vp, ee, kSphFloor));
+            float err;
+            const float det = sph_test(rec[s], e, ee, &err);
             const bool in = (uint32_t)(s * G) + sub < Tl;
             in_m[s] = ballot(in && det > err);
             un[s] = in && !(fabsf(det) > err);
@@ -876,7 +834,7 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
                 break;
             }
             wave_lds_sync();
-            if (sub < nb) L.rec[sub] = SphRec{make_rec(pack_tet(pi, mc, mn), e, E[mc], E[mn]), 0};
+            if (sub < nb) L.rec[sub] = SphRec{sph_rec(pack_tet(pi, mc, mn), e, E[mc], E[mn]), 0};
             wave_lds_sync();
             auto take = [&](int s) {
                 const uint32_t p = (uint32_t)(s * G) + sub;

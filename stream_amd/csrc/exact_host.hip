@@ -1,6 +1,6 @@
-// Host evaluation of the device exact stage (predicates.hpp): the same
-// expansion arithmetic, compiled for the host, for verification against
-// exact rational arithmetic without a GPU.
+// Host evaluation of the device exact stage and of the sphere test
+// (predicates.hpp): the same arithmetic, compiled for the host, for
+// verification against exact rational arithmetic without a GPU.
 #include <vector>
 
 #include "predicates.hpp"
@@ -36,6 +36,24 @@ int32_t Stream_exact_sign_host(int32_t kind, int32_t fp64, const void* pts, int3
         *sign = fp64 ? stream_amd::exact_sign<double>(kind, (const double*)pts, &over)
                      : stream_amd::exact_sign<float>(kind, (const float*)pts, &over);
         if (over) throw std::runtime_error("exact stage workspace exhausted");
+    });
+}
+
+// The FP32 sphere test of (p, b, c, d) against e (5 x 3 doubles), coordinates
+// scaled for the given alpha: 1 when it certifies that e lies inside, -1
+// outside, 0 when it certifies nothing.  The sign is that of -insphere.
+int32_t Stream_sphere_sign_host(const double* pts, double alpha, int32_t* sign) {
+    return stream_amd::guarded([&] {
+        if (!pts || !sign) throw std::invalid_argument("Stream_sphere_sign_host: null argument");
+        const double scale = stream_amd::sph_scale(alpha);
+        float4 q[4];
+        for (int k = 0; k < 4; ++k) {
+            const double* c = pts + 3 * (k + 1);
+            q[k] = stream_amd::sph_point((c[0] - pts[0]) * scale, (c[1] - pts[1]) * scale, (c[2] - pts[2]) * scale);
+        }
+        float err;
+        const float det = stream_amd::sph_test(stream_amd::sph_rec(0u, q[0], q[1], q[2]), q[3], q[3].w * q[3].w, &err);
+        *sign = det > err ? 1 : (-det > err ? -1 : 0);
     });
 }
 

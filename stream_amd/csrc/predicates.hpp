@@ -393,4 +393,68 @@ __host__ __device__ __noinline__ int insphere_exact(const S* a, const S* b, cons
     return acc.sign();
 }
 
+// ---------------------------------------------------------------------------
+// Sphere test of a star: the insphere sign of many points against a
+// tetrahedron (p, b, c, d) that is kept, certified in FP32.  With p as origin
+// the value is e.W - V |e|^2, W = |b|^2 cxd + |c|^2 dxb + |d|^2 bxc and V =
+// b.(cxd); W, V and the factors wp, vp of the error bound are formed once per
+// tetrahedron.  Coordinates are relative to p, divided by a power of two near
+// alpha and rounded to FP32 (from FP32 and FP64 nodes alike).  Each monomial
+// sees at most 21 roundings and the bound takes 24 (kSphBound); the sums of
+// absolute monomials are bounded by the lengths: a component of |c||x||d| by
+// |c| |d|, so W's by Q (|b| + |c| + |d|) and V's by sqrt(3) Q, Q = |b| |c| |d|.
+// A point beyond kSphRange or nearer than kSphNear is NaN and certifies nothing.
+// Between these kSphFloor covers underflow: a length, and its square, keep their
+// relative accuracy, so that a bound vanishes only where its terms do (a product
+// that loses 2^-150 gets factors of at most 5e21 afterwards: 4e-24 each).  With
+// nearer points the length underflowed while the products with infinity nodes
+// did not, and wrong signs were certified.  A certified sign is the exact sign.
+// ---------------------------------------------------------------------------
+constexpr float kSphBound = 1.7320509f * 24.0f * 5.9604644775390625e-08f;
+constexpr float kSphFloor = 1e-20f;
+constexpr float kSphRange = 1e7f;
+constexpr float kSphNear = 1e-15f;
+
+struct SphReg {
+    float wx, wy, wz, v, wp, vp;
+    uint32_t w;  // the caller's name for the tetrahedron
+};
+
+__host__ __device__ __forceinline__ double sph_scale(double alpha) {
+    return (alpha > 0.0 && alpha < 1e300) ? ldexp(1.0, -ilogb(alpha)) : 1.0;
+}
+// A point by its scaled coordinates relative to p; w = its length.
+__host__ __device__ __forceinline__ float4 sph_point(double x, double y, double z) {
+    float4 e;
+    e.x = (float)x;
+    e.y = (float)y;
+    e.z = (float)z;
+    e.w = sqrtf(fmaf(e.x, e.x, fmaf(e.y, e.y, e.z * e.z)));
+    if (!(fmaxf(fabsf(e.x), fmaxf(fabsf(e.y), fabsf(e.z))) <= kSphRange && e.w >= kSphNear)) e.x = e.w = NAN;
+    return e;
+}
+// |c|^2 dxb + |d|^2 bxc = b x (|d|^2 c - |c|^2 d)
+__host__ __device__ __forceinline__ SphReg sph_rec(uint32_t w, const float4& b, const float4& c, const float4& d) {
+    const float x = fmaf(c.y, d.z, -(c.z * d.y)), y = fmaf(c.z, d.x, -(c.x * d.z)), z = fmaf(c.x, d.y, -(c.y * d.x));
+    const float bb = b.w * b.w, cc = c.w * c.w, dd = d.w * d.w;
+    const float gx = fmaf(dd, c.x, -(cc * d.x)), gy = fmaf(dd, c.y, -(cc * d.y)), gz = fmaf(dd, c.z, -(cc * d.z));
+    const float q = kSphBound * (b.w * c.w) * d.w;
+    SphReg r;
+    r.wx = fmaf(bb, x, fmaf(b.y, gz, -(b.z * gy)));
+    r.wy = fmaf(bb, y, fmaf(b.z, gx, -(b.x * gz)));
+    r.wz = fmaf(bb, z, fmaf(b.x, gy, -(b.y * gx)));
+    r.v = fmaf(b.x, x, fmaf(b.y, y, b.z * z));
+    // sum |e_k| <= sqrt(3) |e|
+    r.wp = q * (b.w + c.w + d.w);
+    r.vp = q;
+    r.w = w;
+    return r;
+}
+// The value for e (ee = its length squared): e lies inside where it exceeds
+// *err, outside where it is below -*err.
+__host__ __device__ __forceinline__ float sph_test(const SphReg& r, const float4& e, float ee, float* err) {
+    *err = fmaf(r.wp, e.w, fmaf(r.vp, ee, kSphFloor));
+    return fmaf(e.x, r.wx, fmaf(e.y, r.wy, fmaf(e.z, r.wz, -(ee * r.v))));
+}
+
 }  // namespace stream_amd

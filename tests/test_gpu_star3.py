@@ -3,7 +3,8 @@ bit for bit against the CPU oracle: node counts around a wavefront's four
 nodes, candidate lists from none to the clamped 124 (nodes that wait for room
 in the candidate pool), stars beyond 32 and beyond 64 tetrahedra, cavities
 beyond 14 and 32 and walks that the step cap stops, coordinates far from and
-close to 1 (FP32 tests that only the FP64 filter decides)."""
+close to 1 (FP32 tests that only the FP64 filter decides), and a pair of nodes
+that all but coincide beside infinity nodes at hundreds of alpha."""
 import numpy as np
 import pytest
 
@@ -31,6 +32,12 @@ def _cloud(name):
         return np.random.default_rng(k).random((k, 3)), 0.35 / k ** (1 / 3)
     if kind == "ball":
         return _ball(k, k), 3.0
+    if kind == "twin":  # of the origin, at 2e-23 alpha, in a box of 1,200 alpha
+        rng = np.random.default_rng(k)
+        pts = rng.uniform(-1, 1, (60, 3))
+        pts[30:, 1] = pts[30:, 2] * (1 + 1e-7 * rng.standard_normal(30))  # almost in a plane with the pair
+        box = 600.0 * np.array([[x, y, z] for x in (-1, 1) for y in (-1, 1) for z in (-1, 1)])
+        return np.concatenate([[[0.0, 0.0, 0.0], [-1e-23, 1.3e-23, 1.3e-23]], pts, box]), 1.0
     if kind == "dense":  # alpha well above the spacing: clamped lists
         return np.random.default_rng(k).random((k, 3)), 1.9 / k ** (1 / 3)
     pts, al = clouds.sloshing_tank_scaled(k, 3)
@@ -43,7 +50,7 @@ def _cloud(name):
     ("random-124", 1.0, 0.0), ("random-127", 1.0, 0.0), ("sparse-301", 1.0, 0.0), ("ball-17", 1.0, 0.0),
     ("ball-34", 1.0, 0.0), ("ball-35", 1.0, 0.0), ("ball-60", 1.0, 0.0), ("ball-123", 1.0, 0.0),
     ("dense-1500", 1.0, 0.0), ("dense-400", 2.0 ** -9, 0.0), ("dense-400", 2.0 ** 20, 0.0),
-    ("dense-400", 1.0, 300.0), ("tank-9000", 1.0, 0.0)])
+    ("dense-400", 1.0, 300.0), ("tank-9000", 1.0, 0.0), ("twin-1", 1.0, 0.0), ("twin-5", 1.0, 0.0)])
 def test_outputs_match_oracle(name, scale, offset, dtype):
     from stream_amd.mesh import AlphaShape3D
 
