@@ -286,9 +286,10 @@ template <class S> __device__ __forceinline__ void empty_star(const Ash3Args<S>&
 }
 
 // Local Delaunay of node tid's star + alpha filter (cpp:380-682) by one
-// wavefront, every undecided sign through the exact stage.  A lane tests the
-// tetrahedra at its positions (each is tested once per insertion, and its
-// result depends on it and the point alone, so the order is free); lane 0
+// wavefront, what the FP64 filter leaves undecided through the exact stage
+// (queue[2] counts the nodes that need it; the others are here for space).  A
+// lane tests the tetrahedra at its positions (each is tested once per insertion,
+// and its result depends on it and the point alone, so the order is free); lane 0
 // evaluates the undecided ones, with the expansion in LDS.  Removal and
 // re-triangulation run on the flags, on every lane alike.
 template <class S> struct Exact3Lds {
@@ -319,7 +320,7 @@ template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, u
         p[2] = L.x[j][2];
     };
     uint32_t Tlast = 4;
-    bool over = false;
+    bool over = false, needed = false;
     for (uint32_t pi = kNInf3D; pi < ncand; ++pi) {
         S pe0[3];
         corner(pi, pe0);
@@ -339,9 +340,27 @@ template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, u
                 S err;
                 det = -insphere_filter(pa0, pb, pc, pd, pe0, &err);
                 undecided = !((det > err) || (-det > err));
+                if constexpr (sizeof(S) == sizeof(float)) {
+                    if (undecided) {
+                        double q[5][3];
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            q[0][k] = pa0[k];
+                            q[1][k] = pb[k];
+                            q[2][k] = pc[k];
+                            q[3][k] = pd[k];
+                            q[4][k] = pe0[k];
+                        }
+                        double e2;
+                        const double d2 = -insphere_filter(q[0], q[1], q[2], q[3], q[4], &e2);
+                        undecided = !((d2 > e2) || (-d2 > e2));
+                        det = d2 > 0.0 ? (S)1 : (S)-1;
+                    }
+                }
             }
             // one undecided lane after the other: the workspace is shared
             uint64_t u = __builtin_amdgcn_ballot_w64(undecided);
+            needed |= u != 0;
             for (; u; u &= u - 1) {
                 if (lane == (uint32_t)__builtin_ctzll(u)) {
                     double* ws = L.ws;
@@ -460,6 +479,7 @@ template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, u
         wave_lds_sync();
     }
     if (over) raise_flag(a.flags, kErrCapacity);
+    if (needed && lane == 0) atomicAdd(&a.queue[2], 1u);
     // alpha filter (cpp:590-682): kept tetrahedra count at their corners; this
     // node's own ones come first, a dropped or foreign one giving its position
     // to the last one that is left
@@ -550,8 +570,7 @@ template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, u
 //   new     One lane per new tetrahedron computes its W, V and bounds; the
 //           lane that holds the position picks them up through LDS.
 //
-// A star that outgrows 64 positions goes to the exact kernel (queue[2] counts
-// these).
+// A star that outgrows 64 positions goes to the exact kernel.
 //
 // Bound: instruction issue (364 vector and 264 scalar instructions per
 // insertion of a wavefront's four nodes, three quarters of the vector issue
@@ -994,10 +1013,7 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
         Tl = end;
     }
     if (redo) {
-        if (sub == 0) {
-            a.queue[kQueueIds + atomicAdd(&a.queue[0], 1u)] = tid;
-            if (redo == 2) atomicAdd(&a.queue[2], 1u);
-        }
+        if (sub == 0) a.queue[kQueueIds + atomicAdd(&a.queue[0], 1u)] = tid;
         return;
     }
     // alpha filter: kept tetrahedra count at their corners; this node's own
@@ -1236,7 +1252,7 @@ template <class S> void Ash3D<S>::compute(hipStream_t s) {
 }
 
 template <class S> uint32_t Ash3D<S>::n_exact_nodes() {
-    return computed ? read_scalar(queue.p) - read_scalar(queue.p + 2) : 0u;
+    return computed ? read_scalar(queue.p + 2) : 0u;
 }
 template <class S> uint32_t Ash3D<S>::n_over_cap() { return computed ? read_scalar(queue.p + 1) : 0u; }
 

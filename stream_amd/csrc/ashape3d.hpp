@@ -46,7 +46,7 @@ template <class S> struct Ash3D {
     DBuf<uint8_t> node_is_bnd, nelem, nelem_out;
     DBuf<uint32_t> neig, elemglob;
     DBuf<uint8_t> edge_is_bnd;
-    DBuf<uint32_t> queue;   // counts: redone, candidate overflows, redone for space; then node ids
+    DBuf<uint32_t> queue;   // counts: redone, candidate overflows, exact stage needed; then node ids
     DBuf<uint64_t> scan_ws;
     uint32_t n_elems_ = 0, n_edges_ = 0;
     bool inited = false, computed = false;

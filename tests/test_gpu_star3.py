@@ -4,7 +4,8 @@ nodes, candidate lists from none to the clamped 124 (nodes that wait for room
 in the candidate pool), stars beyond 32 and beyond 64 tetrahedra, cavities
 beyond 14 and 32 and walks that the step cap stops, coordinates far from and
 close to 1 (FP32 tests that only the FP64 filter decides), and a pair of nodes
-that all but coincide beside infinity nodes at hundreds of alpha."""
+that all but coincide beside infinity nodes at hundreds of alpha; and the count
+of the nodes that needed the exact stage."""
 import numpy as np
 import pytest
 
@@ -72,3 +73,27 @@ def test_outputs_match_oracle(name, scale, offset, dtype):
     if dtype == np.float64 and offset == 0.0:
         # room alone never counts as an exact evaluation
         assert a.get_nexact() <= o["n_exact_calls"]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [70, 90])
+def test_exact_nodes_are_counted_whatever_else_they_need(n, dtype):
+    """Five cospherical nodes, a centre and four of its sphere on one circle, and
+    n more of the sphere in general position: these five need the exact stage,
+    the centre's star outgrows 64 tetrahedra as well."""
+    from stream_amd.mesh import AlphaShape3D
+
+    four = np.array([[0.25, 0.125, 0.9375], [-0.25, 0.125, 0.9375], [0.25, -0.125, 0.9375], [-0.25, -0.125, 0.9375]])
+    rng = np.random.default_rng(n)
+    v = rng.standard_normal((40 * n, 3))
+    v *= (np.linalg.norm(four[0]) * (1.0 + 1e-3 * rng.random(len(v))) / np.linalg.norm(v, axis=1))[:, None]
+    v = v[v[:, 2] < 0.7][:n]  # the circle stays empty
+    pts = np.concatenate([np.zeros((1, 3)), four, v]).astype(dtype)
+    al = np.full(len(pts), 3.0, dtype)
+    print(f"[star3] exact nodes n={n} {np.dtype(dtype).name}", flush=True)
+    a = AlphaShape3D(dtype=dtype, morton_bits=21)
+    a.set_nodes(pts, al)
+    a.compute()
+    o = ol.ashape3d(pts, al, bits=21, dtype=dtype)
+    assert np.array_equal(a.get_elem(), o["elem"])
+    assert o["n_exact_calls"] > 0 and a.get_nexact() == 5
