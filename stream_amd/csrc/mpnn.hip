@@ -901,18 +901,23 @@ GemmArgs gargs(uint32_t n, const float* x0, uint32_t ld0, const uint16_t* wt, fl
     return a;
 }
 
+// Rows per block of the weight-gradient products (32-row stages).
+// Bound: the latency of a block's 32-row stages, so as few of them per block
+// as kDwGrid allows: 256 rows per block (one block per CU at 65k nodes) took
+// 87, 67 and 104 us per product, 64 rows 32, 24 and 42 us; small graphs gain
+// most (a gradient on 2,400 nodes 838 -> 510 us).  Beyond kDwGrid blocks the
+// partials' traffic costs more (160k nodes: 2.41 ms at 1,000 blocks, 2.52 at
+// 1,667).
+uint32_t dw_rows(uint32_t n) {
+    const uint32_t rpb = (n + kDwGrid - 1) / kDwGrid;
+    return rpb ? (rpb + 31) / 32 * 32 : 32;
+}
+uint32_t dw_blocks(uint32_t n) { return n ? (n + dw_rows(n) - 1) / dw_rows(n) : 1; }
+
 template <int K, int K0, int N, bool BIAS>
 void run_dw(uint32_t n, const float* x0, uint32_t ld0, const float* x1, uint32_t ld1, const float* dy,
             uint32_t lddy, float* partial, float* dst, hipStream_t s) {
-    // Bound: the latency of a block's 32-row stages, so as few of them per block
-    // as kDwGrid allows: 256 rows per block (one block per CU at 65k nodes) took
-    // 87, 67 and 104 us per product, 64 rows 32, 24 and 42 us; small graphs gain
-    // most (a gradient on 2,400 nodes 838 -> 510 us).  Beyond kDwGrid blocks the
-    // partials' traffic costs more (160k nodes: 2.41 ms at 1,000 blocks, 2.52 at
-    // 1,667).
-    uint32_t rpb = (n + kDwGrid - 1) / kDwGrid;
-    rpb = rpb ? (rpb + 31) / 32 * 32 : 32;
-    const uint32_t nb = n ? (n + rpb - 1) / rpb : 1;
+    const uint32_t rpb = dw_rows(n), nb = dw_blocks(n);
     const uint32_t width = K * N + (BIAS ? N : 0);
     hipLaunchKernelGGL((gemm_dw_kernel<K, K0, N, BIAS>), dim3(nb), dim3(256), 0, s, n, rpb, x0, ld0, x1, ld1, dy,
                        lddy, partial);
@@ -995,9 +1000,6 @@ void MpnnNet::reserve(uint32_t n, uint32_t nnz) {
         y.resize(nnz);
         cap_nnz = nnz;
     }
-    const size_t pw = (size_t)kDwGrid * (3 * kHid * kHid + kHid);
-    const size_t pe = (size_t)kEdgeGrid * kHeadPart;
-    partials.resize(pw > pe ? pw : pe);
     lpart.resize(2ull * 4096);
     lsc.resize(4);
 }
@@ -1040,6 +1042,9 @@ void MpnnNet::backward(const MpnnGraph& g, hipStream_t s) {
     const uint32_t n = g.n;
     if (!n) return;
     const unsigned eg = blocks_for(n, 4, kEdgeGrid);
+    // of the blocks that this graph uses: 5 MB at 2,400 nodes, 63 MB from 41k on
+    const size_t pw = (size_t)dw_blocks(n) * (3 * kHid * kHid + kHid), pe = (size_t)eg * kHeadPart;
+    partials.resize(pw > pe ? pw : pe);
     float* G = grad.p;
     hipLaunchKernelGGL(head_bwd_kernel, dim3(eg), dim3(256), 0, s, n, g.row, g.col, g.val, g.dpos.p, g.tr.p, g.bnd,
                        g.efeat.p, RSD.p, wb.p, w.p, gval.p, od.p, y.p, lsc.p, dRSD.p, partials.p);

@@ -43,3 +43,29 @@ def test_gradient_matches_oracle(n):
     # way (2^-8 of one value in a few tens of thousands)
     assert abs(loss - ref_loss) <= 1e-3 * max(1.0, abs(ref_loss))
     assert np.linalg.norm(grad - ref) <= 1e-2 * np.linalg.norm(ref)
+
+
+def test_partials_take_the_graph_s_own_blocks():
+    """Workspace for the block partials: none without a gradient, then that of the
+    graph's own blocks (75 x 12,352 floats for 2,400 nodes)."""
+    import gc
+
+    import stream_amd
+    from stream_amd.learned import PrecLearned
+
+    n = 2400
+    print(f"[partials] workspace n={n}", flush=True)
+    row, col, val, xy, bnd = _chain_lattice(n)
+    net = PrecLearned(mpnn.init_params(7))
+    gc.collect()  # other tests' networks
+    net.set_system(row, col, val, xy, bnd)
+    net.forward()
+    before = stream_amd.device_bytes()["current"]
+    net.gradient()
+    assert stream_amd.device_bytes()["current"] - before == 4 * 75 * (3 * 64 * 64 + 64)
+    # activations and their gradients take 1,856 floats a node
+    net2 = PrecLearned(mpnn.init_params(7))
+    net2.set_system(row, col, val, xy, bnd)
+    before = stream_amd.device_bytes()["current"]
+    net2.forward()
+    assert stream_amd.device_bytes()["current"] - before < 1.2 * 4 * 1856 * n
