@@ -15,7 +15,8 @@
 // minus the four infinity nodes), local tetrahedra (u32 packing three u8
 // local ids, CAP 256 >= 2*124 + 4 for a star of 124 link vertices) and
 // per-candidate counts (u8).  The insertion itself runs on registers and LDS,
-// 16 lanes per node; only the exact redo works in the slab.
+// 16 lanes per node, or a wavefront in the exact redo; the slab receives the
+// kept tetrahedra and the counts.
 #pragma once
 #include "lbvh.hpp"
 
@@ -27,7 +28,7 @@ constexpr uint32_t kCand3D = 124;    // real candidates per node
 constexpr uint32_t kTet3D = 256;     // local tetrahedra per node
 constexpr uint32_t kCycle3D = 128;   // local ids (4 infinity + 124)
 constexpr uint32_t kExactWaves3D = 4096;  // wavefronts of the exact redo (one queued node each at a time)
-constexpr uint32_t kExactWs3D = 512;  // doubles per lane (expansion components)
+constexpr uint32_t kExactWs3D = 512;  // doubles per wavefront of the exact redo (expansion components)
 
 __host__ __device__ inline size_t slab3(uint32_t t, uint32_t j, uint32_t cap) {
     return ((size_t)(t >> 6) * cap + j) * 64 + (t & 63u);

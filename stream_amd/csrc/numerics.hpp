@@ -17,8 +17,9 @@
 // the steps.  The diagonal is a separate array.  CSR stays the interchange
 // format (reference DeviceCSR, assembly output, FP64 true residuals).
 //
-// CG keeps every scalar on the device.  On small Jacobi systems an iteration
-// is one kernel (cg1_kernel, rule in cg1_threads), else two:
+// CG keeps every scalar on the device.  On small Jacobi systems whose rows are
+// not wide an iteration is one kernel (cg1_kernel, rule in cg1_threads), else
+// two:
 //   dir    : d = z + beta d_old on the own row, q = A d with neighbour
 //            entries of d recomputed from the interleaved {z, d_old} pair
 //            (one load per neighbour), partial d.q;
