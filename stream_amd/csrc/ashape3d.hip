@@ -813,7 +813,10 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
                     const bool joins = (o0 && (o1 || o2 || !(mz & disc))) || (o1 && (o2 || !(mx & disc))) ||
                                        (o2 && !(my & disc));
                     const uint32_t best = group_min(joins ? key : ~0u);
-                    if (best == ~0u) break;
+                    if (best == ~0u) {
+                        first = kEmpty;  // no disc: refused below
+                        break;
+                    }
                     const uint32_t win = best & 15u;
                     disc |= 1u << win;
                     --left;
@@ -846,9 +849,10 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
             const uint32_t again = group_bits(ballot(sub != 0 && mc == first), grp) & ~1u;
             const uint32_t nb = again ? (uint32_t)__builtin_ctz(again) : (uint32_t)G;
             end = m + nb;
-            // (a proper boundary has R + 2 edges, less two per corner inside)
-            if (group_bits(ballot(sub + 1 == nb && mn != first), grp) || nb > R + 2 || ((nb ^ R) & 1u) ||
-                end > kStarTets) {
+            // (a proper boundary has R + 2 edges, less two per corner inside, and
+            // its corners went in before pi: what a broken one reads is no id)
+            if (group_bits(ballot(sub < nb && (mc >= pi || (sub + 1 == nb && mn != first))), grp) || nb > R + 2 ||
+                ((nb ^ R) & 1u) || end > kStarTets) {
                 redo = 2;
                 break;
             }
@@ -987,7 +991,7 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
             wave_lds_sync();
             uint32_t c = first;
             do {
-                if (c >= kCycle3D || end >= kStarTets) {
+                if (c >= pi || end >= kStarTets) {
                     redo = 2;
                     break;
                 }

@@ -4,8 +4,8 @@ nodes, candidate lists from none to the clamped 124 (nodes that wait for room
 in the candidate pool), stars beyond 32 and beyond 64 tetrahedra, cavities
 beyond 14 and 32 and walks that the step cap stops, coordinates far from and
 close to 1 (FP32 tests that only the FP64 filter decides), and a pair of nodes
-that all but coincide beside infinity nodes at hundreds of alpha; and the count
-of the nodes that needed the exact stage."""
+that all but coincide beside infinity nodes at hundreds of alpha; the count of the
+nodes that needed the exact stage; and nodes that coincide, which are refused."""
 import numpy as np
 import pytest
 
@@ -97,3 +97,25 @@ def test_exact_nodes_are_counted_whatever_else_they_need(n, dtype):
     o = ol.ashape3d(pts, al, bits=21, dtype=dtype)
     assert np.array_equal(a.get_elem(), o["elem"])
     assert o["n_exact_calls"] > 0 and a.get_nexact() == 5
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_coinciding_nodes_are_refused(dtype):
+    """A star of coinciding points has no order to break ties by: its cavity's
+    boundary does not close, and the node ends there (an id of the open boundary
+    must not index anything).  The handle computes the next cloud."""
+    from stream_amd import StreamError
+    from stream_amd.mesh import AlphaShape3D
+
+    print(f"[star3] coinciding nodes {np.dtype(dtype).name}", flush=True)
+    rng = np.random.default_rng(10)
+    a = AlphaShape3D(dtype=dtype, morton_bits=21)
+    pts = np.repeat(rng.random((40, 3)), 2, axis=0).astype(dtype)
+    a.set_nodes(pts, np.full(len(pts), 0.4, dtype))
+    with pytest.raises(StreamError, match="capacity"):
+        a.compute()
+    pts = np.ascontiguousarray(pts[::2])
+    al = np.full(len(pts), 0.4, dtype)
+    a.set_nodes(pts, al)
+    a.compute()
+    assert np.array_equal(a.get_elem(), ol.ashape3d(pts, al, bits=21, dtype=dtype)["elem"])
