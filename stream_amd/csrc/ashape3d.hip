@@ -588,6 +588,14 @@ constexpr uint32_t kWalkFree = 14;  // R (R - 1) / 2 <= 100, and R + 2 new ones 
 // node are usual; 448 bring a wavefront's LDS to 10 KB, four per SIMD.
 constexpr uint32_t kStarPool = 448;
 
+// Consecutive nodes share candidates and slab lines, so an XCD (the blocks go to
+// the 8 in turn) takes runs of this many blocks, 256 nodes.  One contiguous eighth
+// of the nodes each left the XCDs unequal loads: 20,000 nodes of 124 candidates in
+// a dense cluster beside 20,000 ordinary ones 7.8 ms (4.9 now), a tank of 299,000
+// 4.05 (3.72), the 2M one 26.6 (24.6).  Shorter runs share less (100,000 uniform
+// nodes 0.68 ms, as before; 0.69 with 16 blocks).
+constexpr uint32_t kStarRun = 64;
+
 struct alignas(16) SphRec {
     SphReg r;
     uint32_t pos;  // where it comes from
@@ -1076,16 +1084,14 @@ __device__ __forceinline__ void star3_node(const Ash3Args<S>& a, uint32_t tid, u
 
 
 template <class S>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void star3_kernel(
-    Ash3Args<S> a, uint32_t blocks_per_xcd) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void star3_kernel(Ash3Args<S> a) {
     constexpr uint32_t G = kStarLanes;
     constexpr uint32_t NPW = 64 / G;
     __shared__ float4 pool[kStarPool];
     __shared__ Star3Lds lds[NPW];
     const uint32_t sub = threadIdx.x % G, grp = threadIdx.x / G;
-    // consecutive nodes share candidates and slab lines: one XCD (blocks go to
-    // the XCDs in turn) takes a contiguous range of them
-    const uint32_t blk = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
+    const uint32_t q = blockIdx.x >> 3;  // of this XCD's blocks
+    const uint32_t blk = (q / kStarRun * 8 + (blockIdx.x & 7u)) * kStarRun + q % kStarRun;
     const uint32_t tid = blk * NPW + grp;
     const uint32_t n = a.n;
     const uint32_t ncand = tid < n ? a.nineig[tid] : 0u;
@@ -1114,8 +1120,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 }
 
 template <class S> void launch_star3(const Ash3Args<S>& a, hipStream_t s) {
-    const uint32_t blocks = (a.n + 64 / kStarLanes - 1) / (64 / kStarLanes), per_xcd = (blocks + 7) / 8;
-    hipLaunchKernelGGL((star3_kernel<S>), dim3(8 * per_xcd), dim3(64), 0, s, a, per_xcd);
+    constexpr uint32_t round = 8 * kStarRun;
+    const uint32_t blocks = (a.n + 64 / kStarLanes - 1) / (64 / kStarLanes);
+    hipLaunchKernelGGL((star3_kernel<S>), dim3((blocks + round - 1) / round * round), dim3(64), 0, s, a);
 }
 
 // One queued node per wavefront (the block is one wavefront): the exact

@@ -1,6 +1,6 @@
 """The 16-lane local Delaunay of the 3D alpha-shape at the edges of its rules,
 bit for bit against the CPU oracle: node counts around a wavefront's four
-nodes, candidate lists from none to the clamped 124 (nodes that wait for room
+nodes, an XCD's 256 and the 2,048 of all, candidate lists from none to the clamped 124 (nodes that wait for room
 in the candidate pool), stars beyond 32 and beyond 64 tetrahedra, cavities
 beyond 14 and 32 and walks that the step cap stops, coordinates far from and
 close to 1 (FP32 tests that only the FP64 filter decides), and a pair of nodes
@@ -39,6 +39,9 @@ def _cloud(name):
         pts[30:, 1] = pts[30:, 2] * (1 + 1e-7 * rng.standard_normal(30))  # almost in a plane with the pair
         box = 600.0 * np.array([[x, y, z] for x in (-1, 1) for y in (-1, 1) for z in (-1, 1)])
         return np.concatenate([[[0.0, 0.0, 0.0], [-1e-23, 1.3e-23, 1.3e-23]], pts, box]), 1.0
+    if kind == "cluster":  # as many nodes again within a hundredth of the box: one-sided clamped lists
+        rng = np.random.default_rng(k)
+        return np.concatenate([rng.random((k, 3)), 0.5 + 0.01 * rng.random((k, 3))]), 1.1 / k ** (1 / 3)
     if kind == "dense":  # alpha well above the spacing: clamped lists
         return np.random.default_rng(k).random((k, 3)), 1.9 / k ** (1 / 3)
     pts, al = clouds.sloshing_tank_scaled(k, 3)
@@ -48,7 +51,8 @@ def _cloud(name):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("name, scale, offset", [
     ("random-4", 1.0, 0.0), ("random-5", 1.0, 0.0), ("random-7", 1.0, 0.0), ("random-33", 1.0, 0.0),
-    ("random-124", 1.0, 0.0), ("random-127", 1.0, 0.0), ("sparse-301", 1.0, 0.0), ("ball-17", 1.0, 0.0),
+    ("random-124", 1.0, 0.0), ("random-127", 1.0, 0.0), ("sparse-255", 1.0, 0.0), ("sparse-257", 1.0, 0.0),
+    ("sparse-2048", 1.0, 0.0), ("sparse-2049", 1.0, 0.0), ("cluster-1500", 1.0, 0.0), ("sparse-301", 1.0, 0.0), ("ball-17", 1.0, 0.0),
     ("ball-34", 1.0, 0.0), ("ball-35", 1.0, 0.0), ("ball-60", 1.0, 0.0), ("ball-123", 1.0, 0.0),
     ("dense-1500", 1.0, 0.0), ("dense-400", 2.0 ** -9, 0.0), ("dense-400", 2.0 ** 20, 0.0),
     ("dense-400", 1.0, 300.0), ("tank-9000", 1.0, 0.0), ("twin-1", 1.0, 0.0), ("twin-5", 1.0, 0.0)])
