@@ -172,11 +172,13 @@ template <class S> __global__ __launch_bounds__(kFillBlock) void fill_group_kern
     }
     if (sub == 0) a.nineig[tid] = kNInf2D + found;
 }
-// Up to here one lane per node leaves the chip waiting for its walks (us, one
-// lane -> 8, FP32 dam-break: 81 -> 28 at 4k nodes, 92 -> 52 at 65k, 111 -> 106
-// at 160k); beyond, what the 8 lanes do for nothing costs more (157 -> 180 at
-// 300k, 489 -> 586 at 1M).
-constexpr uint32_t kFillGroupMax = 196608;
+// Up to here one lane per node leaves the chip waiting for its walks; beyond,
+// what the 8 lanes do for nothing costs more, first where walks are short.  us,
+// one lane -> 8, FP32, alpha 1.2 spacings: 77 -> 30 at 4k nodes, 85 -> 54 at 65k,
+// 95 -> 77 at 98k, 100 -> 105 at 150k, 489 -> 586 at 1M; alpha half a spacing: 51
+// -> 27 at 10k, 54 -> 45 at 65k, 59 -> 56 at 80k, 58 -> 62 at 98k, 61 -> 86 at
+// 150k; FP64 (6 to 15 more) crosses at the same sizes.
+constexpr uint32_t kFillGroupMax = 90112;
 template <class S> void launch_fill(const AshArgs<S>& a, hipStream_t s) {
     if (a.n > kFillGroupMax) {
         hipLaunchKernelGGL((fill_kernel<S>), dim3((a.n + kFillBlock - 1) / kFillBlock), dim3(kFillBlock), 0, s, a);

@@ -34,7 +34,7 @@ def test_alphashape2d_matches_oracle(name, dtype):
     _check(*_cloud(name), dtype, name)
 
 
-@pytest.mark.parametrize("n", [196_608, 196_609])
+@pytest.mark.parametrize("n", [90_112, 90_113])
 def test_both_sides_of_the_rule(n):
     pts = ol.glibc_uniform(n, 2, 7)
     _check(pts, np.float32(1.2 / n ** 0.5), np.float32, f"uniform {n}")
