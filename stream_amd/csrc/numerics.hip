@@ -1515,16 +1515,17 @@ void cg_solve_llt(const DevCsr<double>& A64, const Sell<V>& S, const LowerFactor
 // records' gathers cost more than the second launch.  One block per CU as
 // far as 256 threads allow that: 7.2 against 8.2 us with 512 at 16k.
 // A gather of an entry moves twice the bytes, so wide rows lose what the launch
-// saves.  Lattices in Morton order, 96 iterations with start and end, two
-// kernels -> one.  FP64 at 64k rows: 26 entries per row 17.8 -> 16.6, 54 23.6 ->
-// 23.9, 113 38.2 -> 39.5; at 91k: 11 15.7 -> 14.8, 26 20.7 -> 21.3, 54 27.1 ->
-// 31.7, 182 64.4 -> 84.2.  FP32 at 91k: 26 19.4 -> 16.9, 76 30.4 -> 29.4, 114
-// 39.1 -> 37.5, 182 55.6 -> 55.4; at 195k: 11 17.5 -> 17.2, 26 23.0 -> 23.0, 55
-// 29.7 -> 31.6, 186 75.5 -> 94.9.
+// saves, sooner where neighbours are far apart.  96 iterations with start and end,
+// two kernels -> one, lattices in Morton order and random graphs (r).  FP64 to 65k
+// rows: 26 entries per row 17.8 -> 16.6, 54 23.6 -> 23.9, r 17 24.3 -> 24.7, r 31
+// 32.8 -> 34.3; at 91k and r 100k: 11 15.7 -> 14.8, 26 20.7 -> 21.3, 54 27.1 -> 31.7,
+// r 9 25.6 -> 26.2, r 17 30.7 -> 35.2.  FP32 to 131k: 54 24.8 -> 23.0, r 31 38.5 ->
+// 34.3, r 57 at 65k 32.2 -> 33.4; at 195k: 5 14.9 -> 14.4, 11 17.5 -> 17.2, 55 29.7
+// -> 31.6, r 9 24.0 -> 26.0, r 17 32.0 -> 34.5.
 template <class V> uint32_t cg1_threads(uint32_t n, uint32_t nnz) {
-    constexpr bool wide = sizeof(V) == 8;
-    if (n > (wide ? 256u : 384u) * 512u) return 0;
-    const uint32_t most = wide ? (n <= 65536u ? 40u : 20u) : (n <= 131072u ? 100u : 20u);
+    constexpr bool f64 = sizeof(V) == 8;
+    if (n > (f64 ? 256u : 384u) * 512u) return 0;
+    const uint32_t most = f64 ? (n <= 65536u ? 24u : 12u) : (n <= 131072u ? 40u : 8u);
     if (nnz > (uint64_t)most * n) return 0;
     return n <= 256u * 256u ? 256 : 512;
 }
