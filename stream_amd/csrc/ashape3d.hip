@@ -576,8 +576,8 @@ template <class S> __device__ void local_delaunay3_exact(const Ash3Args<S>& a, u
 // insertion of a wavefront's four nodes, three quarters of the vector issue
 // slots at 4 wavefronts per SIMD).  5 wavefronts (96 registers) spill and are
 // a third slower.  From one lane per node to this: 1,996,920 FP64 nodes 68.7 ->
-// 26.5 ms, 100,000 FP32 ones 2.50 -> 0.69 ms, 20,102 FP32 ones (79 blocks of
-// one lane per node left most of the chip idle) 3.96 -> 0.49 ms.
+// 24.6 ms, 100,000 FP32 ones 2.50 -> 0.68 ms, 20,102 FP32 ones (79 blocks of
+// one lane per node left most of the chip idle) 3.96 -> 0.43 ms.
 constexpr int kStarLanes = 16;
 constexpr uint32_t kStarTets = 64;
 constexpr int kStarSlots = (int)kStarTets / kStarLanes;
